@@ -420,6 +420,15 @@ int nanorts_amd_env_step(void* stream, const nanorts_game* game, nanorts_state s
 int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, int32_t partial, nanorts_env_results results);
 
+/* nanorts_amd_env_step (reset != 0) or nanorts_amd_env_transition (reset == 0)
+ * from the state `from` into the state `state`, whose leaves the call fills:
+ * the input state stays as it is, which is the reference's env.step without
+ * donation (src/nanorts/adapters/jaxmarl/facade.py:107-119).  Each leaf of
+ * `state` is the same buffer as `from`'s or overlaps no leaf of it. */
+int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
+                              int64_t lanes, const int32_t* actions, int32_t partial, int32_t reset,
+                              nanorts_env_results results);
+
 /* The JaxMARL request (src/nanorts/adapters/jaxmarl/env.py:181-184):
  * decode_actions of int32[L][2][C][7] action rows into Commands
  * (src/nanorts/adapters/jaxmarl/actions.py:61-84) and, when `episode_keys`
@@ -543,6 +552,16 @@ int nanorts_amd_seat_step_lanes(void* stream, const nanorts_game* game, nanorts_
                             nanorts_abstract_actions carry, const int32_t* actions, int32_t partial,
                             nanorts_env_results results);
 
+/* The seat step from the state `from`, the carry `carry_from` and (for
+ * per-lane seats; both NULL for the static `learner`) the seats `seats_from`
+ * into `state`, `carry` and `seats`, which the call fills; the inputs stay as
+ * they are.  Buffers as for nanorts_amd_env_step_from. */
+int nanorts_amd_seat_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
+                               int64_t lanes, int32_t strategy, int32_t trained_type, int32_t learner,
+                               const int32_t* seats_from, int32_t* seats, int32_t draw,
+                               nanorts_abstract_actions carry_from, nanorts_abstract_actions carry,
+                               const int32_t* actions, int32_t partial, nanorts_env_results results);
+
 /* The "drawn" rule's seat of each lane's current episode:
  * randint(fold_in(fold_in(environment_root, episode_index), 2**32 - 2), (),
  * 0, 2) into seats int32[L].  Replaces _episode_seat
@@ -616,6 +635,13 @@ int nanorts_amd_gridnet_step(void* stream, const nanorts_game* game, nanorts_sta
  * (src/nanorts/adapters/gridnet/env.py:73-83). */
 int nanorts_amd_gridnet_step_against(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                                  const int32_t* actions, nanorts_commands commands, nanorts_gridnet_results results);
+
+/* The GridNet step (commands NULL) or step_against (player 1 plays
+ * `*commands`) from the state `from` into `state`, as
+ * nanorts_amd_env_step_from. */
+int nanorts_amd_gridnet_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
+                                  int64_t lanes, const int32_t* actions, const nanorts_commands* commands,
+                                  nanorts_gridnet_results results);
 
 /* The synthetic harness's integer uniform-over-legal sampler on the GridNet
  * surface: per-cell actions int32[L][2][H][W][7] from the packed action mask

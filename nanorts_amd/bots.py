@@ -99,6 +99,19 @@ class SeatState:
                          self.seat.clone())
 
 
+    def step_buffers(self, donate: bool) -> tuple["SeatState", "SeatState"]:
+        """(the seat state a step launch reads, the one it writes), as
+        EnvironmentState.step_buffers."""
+        if donate:
+            return self, self
+        tensors = [*(self.carry[f] for f in native.ABSTRACT_FIELDS), self.seat]
+        if not (self.environment_state.is_contiguous and all(t.is_contiguous() for t in tensors)):
+            copied = self.clone()
+            return copied, copied
+        carry = {k: torch.empty_like(v) if k in native.ABSTRACT_FIELDS else v.clone() for k, v in self.carry.items()}
+        return self, SeatState(self.environment_state.successor(), carry, torch.empty_like(self.seat))
+
+
 def _pick(per_agent: dict[str, Any], seat: torch.Tensor) -> Any:
     """_learners (src/nanorts/bots/seat.py:368-375) for per-lane seats: lane
     l's value of player seat[l], for a tensor or an observation record."""
@@ -180,7 +193,7 @@ class SeatEnv:
         if reset_state is not None:
             raise ModelError("step resets finished games to the content's start by itself; reset_state is not taken")
         env = self.env
-        nxt = state if donate else state.clone()
+        before, nxt = state.step_buffers(donate)
         es = nxt.environment_state
         L = es.num_envs
         b = env.bucket
@@ -207,19 +220,23 @@ class SeatEnv:
             _ptr(out["reward"]), _ptr(out["done"]), _ptr(out["terminated"]), _ptr(out["truncated"]),
             _ptr(out["winner"]), _ptr(out["spawn_overflowed"]), _ptr(maps), _ptr(scalars), _ptr(fmaps), _ptr(fscal),
             _ptr(comps), _ptr(out["spawn_overflow"]))
+        seats_from = seats = None
+        current = before.seat
         if self.learner is not None:
-            current = nxt.seat
-            native.check(env.lib.nanorts_amd_seat_step(_stream(), env.dev.ref, es.native(), L, self.bot.strategy,
-                                                   self.bot.trained, self.learner, _carry_struct(nxt.carry),
-                                                   _ptr(acts), env.partial, results), "nanorts_amd_seat_step")
+            if before is not nxt:
+                nxt.seat.copy_(before.seat)
         else:
             if nxt.seat.dtype != torch.int32 or tuple(nxt.seat.shape) != (L,) or not nxt.seat.is_contiguous():
                 raise ModelError(f"the seat state's seat must be a contiguous int32[{L}]")
-            current = nxt.seat.clone()
-            native.check(env.lib.nanorts_amd_seat_step_lanes(_stream(), env.dev.ref, es.native(), L, self.bot.strategy,
-                                                         self.bot.trained, _ptr(nxt.seat), int(self.draw),
-                                                         _carry_struct(nxt.carry), _ptr(acts), env.partial, results),
-                         "nanorts_amd_seat_step_lanes")
+            if before is nxt:
+                current = before.seat.clone()  # the launch may draw the next episode's over it
+            seats_from, seats = _ptr(before.seat), _ptr(nxt.seat)
+        native.check(env.lib.nanorts_amd_seat_step_from(_stream(), env.dev.ref, before.environment_state.native(),
+                                                        es.native(), L, self.bot.strategy, self.bot.trained,
+                                                        self.learner or 0, seats_from, seats, int(self.draw),
+                                                        _carry_struct(before.carry), _carry_struct(nxt.carry),
+                                                        _ptr(acts), env.partial, results),
+                     "nanorts_amd_seat_step_from")
         publish = env._symbolic if env.layout.surface == "symbolic" else env._pixels
         obs = self._learners(publish(maps, scalars), nxt.seat)
         infos: dict[str, Any] = {

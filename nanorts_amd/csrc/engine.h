@@ -636,6 +636,13 @@ NR_DEV void store_scalars(const nanorts_state& s, int64_t l, const Env& e, int l
     }
 }
 
+// The root into row l of `s`, where a step writes another state than the one
+// it read (`from`; the store above leaves the root, which no step changes).
+NR_DEV void store_root(const nanorts_state& from, const nanorts_state& s, int64_t l, const Env& e, int lane) {
+    if (s.environment_root != from.environment_root && lane < 2)
+        s.environment_root[2 * l + lane] = (uint32_t)e.sc[S_ROOT0 + lane];
+}
+
 // Leaves of at most 1024 bytes (one 16-byte vector per lane), 16-byte
 // aligned: every requested leaf is loaded into registers before the first
 // LDS store, so the wave waits on memory once instead of once per leaf.

@@ -1103,10 +1103,17 @@ NR_DEV bool finish_step(const KGame& g, const Hdr& h, const Env& e, int64_t l, i
     return done;
 }
 
-__global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanorts_state s, const int32_t* actions, int32_t partial,
-                           nanorts_env_results r, int32_t reset) {
+// A step reads the state `from` and writes the state `s`: the same rows for a
+// step in place, or the caller's fresh buffers, which a step that leaves its
+// input state alone then fills by itself.  (Copying the 25 leaves first, one
+// device copy apiece, took 25 launches and one more pass over the state: a
+// masks-and-step turn of 64 games on 8x8 ran 207 us with the copies and
+// 130 us without, of 4096 games on 16x16 219 us and 130 us.)  A wave reads its
+// game's rows before it writes any.
+__global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanorts_state from, nanorts_state s,
+                           const int32_t* actions, int32_t partial, nanorts_env_results r, int32_t reset) {
     NR_KERNEL_PROLOGUE
-    load_env(g, s, l, e, LD_ALL, lane);
+    load_env(g, from, l, e, LD_ALL, lane);
     count_units(g, e, lane);
     const int32_t owned = 2 * g.C;
     uint32_t k0 = (uint32_t)uni(e.sc[S_ROOT0]), k1 = (uint32_t)uni(e.sc[S_ROOT1]);
@@ -1162,6 +1169,7 @@ __global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanort
     }
     finish_step(g, hdr, e, l, lane, partial != 0, r, events, fast, reset != 0);
     store_env(g, s, l, e, lane);
+    store_root(from, s, l, e, lane);
     if (fast) {
         const int64_t per = (int64_t)g.cells * 6;
         uint8_t* m0 = r.feature_maps ? r.feature_maps + (l * 2) * per : nullptr;
@@ -1409,12 +1417,16 @@ __global__ __launch_bounds__(256) void k_astar_chain(AstarArgs a) {
 // observations.  The learner is `fixed` for every lane, or seats[l] when
 // `seats` is set; with `draw` a lane whose game ended takes the seat drawn
 // from its next episode's root (N/bots/seat.py:119-123).
-__global__ __launch_bounds__(256) void k_seat_step(KGame g, int64_t lanes, nanorts_state s, BotArgs a, int32_t fixed,
-                                                   int32_t* seats, int32_t draw, const int32_t* actions,
-                                                   int32_t partial, nanorts_env_results r) {
+// The state, the carry and the seats are read from `from`, `carry_from` and
+// `seats_from` and written to `s`, `a.carry` and `seats` (see k_env_step).
+__global__ __launch_bounds__(256) void k_seat_step(KGame g, int64_t lanes, nanorts_state from, nanorts_state s,
+                                                   BotArgs a, BotCarry carry_from, int32_t fixed,
+                                                   const int32_t* seats_from, int32_t* seats, int32_t draw,
+                                                   const int32_t* actions, int32_t partial, nanorts_env_results r) {
     NR_KERNEL_PROLOGUE
-    const int32_t learner = seats ? clampi(uni(seats[l]), 0, 1) : fixed;
-    load_env(g, s, l, e, LD_ALL, lane);
+    const int32_t seat = seats ? uni(seats_from[l]) : fixed;
+    const int32_t learner = clampi(seat, 0, 1);
+    load_env(g, from, l, e, LD_ALL, lane);
     count_units(g, e, lane);
     uint32_t k0 = (uint32_t)uni(e.sc[S_ROOT0]), k1 = (uint32_t)uni(e.sc[S_ROOT1]);
     fold_in(k0, k1, (uint32_t)uni(e.sc[S_EPISODE]));
@@ -1422,7 +1434,7 @@ __global__ __launch_bounds__(256) void k_seat_step(KGame g, int64_t lanes, nanor
     b.base = e.base + a.y.origin;
     b.player = 1 - learner;
     b.block = g.N + b.player * g.C;
-    const int32_t kept = bot_act(g, hdr, e, b, a.y, l, a.carry, a.strategy, a.trained, lane);
+    const int32_t kept = bot_act(g, hdr, e, b, a.y, l, carry_from, a.strategy, a.trained, lane);
     const Layout& y = g.lay;
     const int32_t top = (1 << g.rank_bits) - 1;
     for (int32_t p = lane; p < 2 * g.C; p += kWave) {
@@ -1450,16 +1462,18 @@ __global__ __launch_bounds__(256) void k_seat_step(KGame g, int64_t lanes, nanor
     wave_sync();
     const bool events = r.reward_components != nullptr;
     core_step(g, hdr, e, lane, k0, k1, events);
+    int32_t next_seat = seat;
     if (finish_step(g, hdr, e, l, lane, partial != 0, r, events)) {
         clear_carry(g, l, a.carry, lane);
         if (seats && draw) {
             uint32_t n0 = (uint32_t)uni(e.sc[S_ROOT0]), n1 = (uint32_t)uni(e.sc[S_ROOT1]);
             fold_in(n0, n1, (uint32_t)uni(e.sc[S_EPISODE]));
-            const int32_t next = episode_seat(n0, n1);
-            if (lane == 0) seats[l] = next;
+            next_seat = episode_seat(n0, n1);
         }
     }
+    if (seats && lane == 0) seats[l] = next_seat;
     store_env(g, s, l, e, lane);
+    store_root(from, s, l, e, lane);
     if (r.feature_maps || r.scalars) observe_both(g, hdr, e, l, lane, partial != 0, r.feature_maps, r.scalars);
 }
 
@@ -2445,11 +2459,12 @@ __global__ __launch_bounds__(256) void k_gridnet_observe(KGame g, int64_t lanes,
 // auto-reset and the observation of the post-reset state.  With `against`,
 // step_against (env.py:73-83): player 0's rows are decoded from `actions`
 // ([L][H][W][7]) and player 1 plays the given Commands.
-__global__ __launch_bounds__(256) void k_gridnet_step(KGame g, int64_t lanes, nanorts_state s, GridLayout gy,
-                                                      const int32_t* actions, nanorts_commands given, int32_t against,
-                                                      nanorts_gridnet_results r) {
+// The state is read from `from` and written to `s` (see k_env_step).
+__global__ __launch_bounds__(256) void k_gridnet_step(KGame g, int64_t lanes, nanorts_state from, nanorts_state s,
+                                                      GridLayout gy, const int32_t* actions, nanorts_commands given,
+                                                      int32_t against, nanorts_gridnet_results r) {
     NR_KERNEL_PROLOGUE
-    load_env(g, s, l, e, LD_ALL, lane);
+    load_env(g, from, l, e, LD_ALL, lane);
     count_units(g, e, lane);
     uint32_t k0 = (uint32_t)uni(e.sc[S_ROOT0]), k1 = (uint32_t)uni(e.sc[S_ROOT1]);
     fold_in(k0, k1, (uint32_t)uni(e.sc[S_EPISODE]));
@@ -2507,6 +2522,7 @@ __global__ __launch_bounds__(256) void k_gridnet_step(KGame g, int64_t lanes, na
     er.spawn_overflow = r.spawn_overflow;
     finish_step(g, hdr, e, l, lane, false, er, true);
     store_env(g, s, l, e, lane);
+    store_root(from, s, l, e, lane);
     gridnet_observe(g, hdr, e, l, lane, r.observation, r.observation.planes);
 }
 
@@ -2755,12 +2771,13 @@ const char* nanorts_amd_build_id(void) { return NANORTS_BUILD_ID; }
 const char* nanorts_amd_entries(void) {
     return "nanorts_amd_step,nanorts_amd_step_ffi,nanorts_amd_legality,nanorts_amd_legality_words,nanorts_amd_legality_ffi,"
            "nanorts_amd_avail_actions,nanorts_amd_visible_cells,nanorts_amd_visible_cells_ffi,nanorts_amd_reset_rows_ffi,"
-           "nanorts_amd_observe,nanorts_amd_pixels,nanorts_amd_pixels_from_maps,nanorts_amd_reset_where_done,nanorts_amd_env_step,nanorts_amd_sample_actions,"
+           "nanorts_amd_observe,nanorts_amd_pixels,nanorts_amd_pixels_from_maps,nanorts_amd_reset_where_done,nanorts_amd_env_step,nanorts_amd_env_step_from,nanorts_amd_sample_actions,"
            "nanorts_amd_step_groups,nanorts_amd_step_groups_ffi,nanorts_amd_env_transition,nanorts_amd_decode_actions,nanorts_amd_rollout,"
-           "nanorts_amd_abstraction_act,nanorts_amd_abstraction_act_ffi,nanorts_amd_seat_step,nanorts_amd_seat_rollout,"
+           "nanorts_amd_abstraction_act,nanorts_amd_abstraction_act_ffi,nanorts_amd_seat_step,nanorts_amd_seat_step_from,nanorts_amd_seat_rollout,"
            "nanorts_amd_seat_step_lanes,nanorts_amd_seat_rollout_lanes,nanorts_amd_episode_seats,nanorts_amd_astar_search_ffi,"
            "nanorts_amd_astar_chain_ffi,nanorts_amd_gridnet_decode,nanorts_amd_gridnet_decode_ffi,"
-           "nanorts_amd_gridnet_observe,nanorts_amd_gridnet_step,nanorts_amd_gridnet_step_against,nanorts_amd_gridnet_sample_actions";
+           "nanorts_amd_gridnet_observe,nanorts_amd_gridnet_step,nanorts_amd_gridnet_step_against,nanorts_amd_gridnet_step_from,"
+           "nanorts_amd_gridnet_sample_actions";
 }
 
 const char* nanorts_amd_last_error(void) { return g_error.c_str(); }
@@ -3351,27 +3368,34 @@ int nanorts_amd_reset_where_done(void* stream, const nanorts_game* game, nanorts
     return launch(k_reset, sh, lanes, (hipStream_t)stream, state, done);
 }
 
+// One env.step launch from the state `from` into `state` (see
+// nanorts_amd_env_step_from).
+static int env_step(void* stream, const nanorts_game* game, const nanorts_state& from, const nanorts_state& state,
+                    int64_t lanes, const int32_t* actions, int32_t partial, int32_t reset,
+                    const nanorts_env_results& results, const char* call) {
+    NR_SHAPE(game)
+    NR_STATE(from)
+    NR_STATE(state)
+    if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
+    if (!from.environment_root || !from.episode_index || !state.environment_root || !state.episode_index)
+        return fail(NANORTS_INVALID_ARGUMENT, std::string(call) + " needs environment_root and episode_index");
+    if (reset && !state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
+    return launch(k_env_step, sh, lanes, (hipStream_t)stream, from, state, actions, partial, results, reset);
+}
 int nanorts_amd_env_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes, const int32_t* actions,
                      int32_t partial, nanorts_env_results results) {
-    NR_SHAPE(game)
-    NR_STATE(state)
-    if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
-    if (!state.environment_root || !state.episode_index)
-        return fail(NANORTS_INVALID_ARGUMENT, "env.step needs environment_root and episode_index");
-    if (!state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
-    return launch(k_env_step, sh, lanes, (hipStream_t)stream, state, actions, partial, results, 1);
+    return env_step(stream, game, state, state, lanes, actions, partial, 1, results, "env.step");
 }
-
 int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, int32_t partial, nanorts_env_results results) {
-    NR_SHAPE(game)
-    NR_STATE(state)
-    if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
-    if (!state.environment_root || !state.episode_index)
-        return fail(NANORTS_INVALID_ARGUMENT, "env.step_env needs environment_root and episode_index");
-    return launch(k_env_step, sh, lanes, (hipStream_t)stream, state, actions, partial, results, 0);
+    return env_step(stream, game, state, state, lanes, actions, partial, 0, results, "env.step_env");
 }
-
+int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
+                              int64_t lanes, const int32_t* actions, int32_t partial, int32_t reset,
+                              nanorts_env_results results) {
+    return env_step(stream, game, from, state, lanes, actions, partial, reset != 0, results,
+                    reset ? "env.step" : "env.step_env");
+}
 int nanorts_amd_decode_actions(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, nanorts_command_buffers commands, uint32_t* episode_keys) {
     NR_SHAPE(game)
@@ -3605,20 +3629,23 @@ int nanorts_amd_astar_chain_ffi(void* stream, const void* const* operands, const
     return launch_astar(k_astar_chain, a, (hipStream_t)stream);
 }
 
-static int seat_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes, int32_t strategy,
-                     int32_t trained_type, int32_t learner, int32_t* seats, int32_t draw,
-                     nanorts_abstract_actions carry, const int32_t* actions, int32_t partial,
-                     nanorts_env_results results) {
+static int seat_step(void* stream, const nanorts_game* game, const nanorts_state& from, const nanorts_state& state,
+                     int64_t lanes, int32_t strategy, int32_t trained_type, int32_t learner, const int32_t* seats_from,
+                     int32_t* seats, int32_t draw, const nanorts_abstract_actions& carry_from,
+                     const nanorts_abstract_actions& carry, const int32_t* actions, int32_t partial,
+                     const nanorts_env_results& results) {
     if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
-    if (!state.environment_root || !state.episode_index)
+    if (!from.environment_root || !from.episode_index || !state.environment_root || !state.episode_index)
         return fail(NANORTS_INVALID_ARGUMENT, "the seat step needs environment_root and episode_index");
     if (!state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
     Shape sh;
-    BotArgs a;
+    BotArgs a, before;
     std::string why;
-    if (!bot_args(game, &sh, &a, strategy, trained_type, carry, &why)) return fail(NANORTS_INVALID_ARGUMENT, why);
-    return launch(k_seat_step, sh, lanes, (hipStream_t)stream, state, a, learner, seats, draw, actions, partial,
-                  results);
+    if (!bot_args(game, &sh, &before, strategy, trained_type, carry_from, &why) ||
+        !bot_args(game, &sh, &a, strategy, trained_type, carry, &why))
+        return fail(NANORTS_INVALID_ARGUMENT, why);
+    return launch(k_seat_step, sh, lanes, (hipStream_t)stream, from, state, a, before.carry, learner, seats_from, seats,
+                  draw, actions, partial, results);
 }
 
 int nanorts_amd_seat_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes, int32_t strategy,
@@ -3626,8 +3653,8 @@ int nanorts_amd_seat_step(void* stream, const nanorts_game* game, nanorts_state 
                       int32_t partial, nanorts_env_results results) {
     NR_STATE(state)
     if (learner != 0 && learner != 1) return fail(NANORTS_INVALID_ARGUMENT, "learner must be 0 or 1");
-    return seat_step(stream, game, state, lanes, strategy, trained_type, learner, nullptr, 0, carry, actions, partial,
-                     results);
+    return seat_step(stream, game, state, state, lanes, strategy, trained_type, learner, nullptr, nullptr, 0, carry,
+                     carry, actions, partial, results);
 }
 
 int nanorts_amd_seat_step_lanes(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
@@ -3636,8 +3663,22 @@ int nanorts_amd_seat_step_lanes(void* stream, const nanorts_game* game, nanorts_
                             nanorts_env_results results) {
     NR_STATE(state)
     if (!seats) return fail(NANORTS_INVALID_ARGUMENT, "seats is NULL");
-    return seat_step(stream, game, state, lanes, strategy, trained_type, 0, seats, draw != 0, carry, actions, partial,
-                     results);
+    return seat_step(stream, game, state, state, lanes, strategy, trained_type, 0, seats, seats, draw != 0, carry, carry,
+                     actions, partial, results);
+}
+
+int nanorts_amd_seat_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
+                               int64_t lanes, int32_t strategy, int32_t trained_type, int32_t learner,
+                               const int32_t* seats_from, int32_t* seats, int32_t draw,
+                               nanorts_abstract_actions carry_from, nanorts_abstract_actions carry,
+                               const int32_t* actions, int32_t partial, nanorts_env_results results) {
+    NR_STATE(from)
+    NR_STATE(state)
+    if ((seats_from == nullptr) != (seats == nullptr))
+        return fail(NANORTS_INVALID_ARGUMENT, "seats_from and seats are both set or both NULL");
+    if (!seats && learner != 0 && learner != 1) return fail(NANORTS_INVALID_ARGUMENT, "learner must be 0 or 1");
+    return seat_step(stream, game, from, state, lanes, strategy, trained_type, learner, seats_from, seats,
+                     seats && draw != 0, carry_from, carry, actions, partial, results);
 }
 
 int nanorts_amd_episode_seats(void* stream, const uint32_t* environment_root, const uint32_t* episode_index, int64_t lanes,
@@ -3884,11 +3925,18 @@ int nanorts_amd_gridnet_observe(void* stream, const nanorts_game* game, nanorts_
     return launch(k_gridnet_observe, sh, lanes, (hipStream_t)stream, state, obs);
 }
 
-int nanorts_amd_gridnet_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
-                         const int32_t* actions, nanorts_gridnet_results results) {
+// One GridNet step launch from the state `from` into `state`; player 1 plays
+// `given` when it is not NULL.
+static int gridnet_step(void* stream, const nanorts_game* game, const nanorts_state& from, const nanorts_state& state,
+                        int64_t lanes, const int32_t* actions, const nanorts_commands* given,
+                        const nanorts_gridnet_results& results) {
+    NR_STATE(from)
     NR_STATE(state)
     if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
-    if (!state.environment_root || !state.episode_index)
+    if (given && (!given->kind || !given->direction || !given->none_duration || !given->target_cell ||
+                  !given->produced_type || !given->request_order))
+        return fail(NANORTS_INVALID_ARGUMENT, "a Commands operand is NULL");
+    if (!from.environment_root || !from.episode_index || !state.environment_root || !state.episode_index)
         return fail(NANORTS_INVALID_ARGUMENT, "the GridNet step needs environment_root and episode_index");
     if (!state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
     Shape sh;
@@ -3897,25 +3945,24 @@ int nanorts_amd_gridnet_step(void* stream, const nanorts_game* game, nanorts_sta
     if (!shape_for_gridnet(game, &sh, &gy, &why) || !gridnet_obs_valid(results.observation, &why))
         return fail(NANORTS_INVALID_ARGUMENT, why);
     const nanorts_commands none = {};
-    return launch(k_gridnet_step, sh, lanes, (hipStream_t)stream, state, gy, actions, none, 0, results);
+    return launch(k_gridnet_step, sh, lanes, (hipStream_t)stream, from, state, gy, actions, given ? *given : none,
+                  given ? 1 : 0, results);
+}
+
+int nanorts_amd_gridnet_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
+                         const int32_t* actions, nanorts_gridnet_results results) {
+    return gridnet_step(stream, game, state, state, lanes, actions, nullptr, results);
 }
 
 int nanorts_amd_gridnet_step_against(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                                  const int32_t* actions, nanorts_commands commands, nanorts_gridnet_results results) {
-    NR_STATE(state)
-    if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
-    if (!commands.kind || !commands.direction || !commands.none_duration || !commands.target_cell ||
-        !commands.produced_type || !commands.request_order)
-        return fail(NANORTS_INVALID_ARGUMENT, "a Commands operand is NULL");
-    if (!state.environment_root || !state.episode_index)
-        return fail(NANORTS_INVALID_ARGUMENT, "the GridNet step needs environment_root and episode_index");
-    if (!state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
-    Shape sh;
-    GridLayout gy;
-    std::string why;
-    if (!shape_for_gridnet(game, &sh, &gy, &why) || !gridnet_obs_valid(results.observation, &why))
-        return fail(NANORTS_INVALID_ARGUMENT, why);
-    return launch(k_gridnet_step, sh, lanes, (hipStream_t)stream, state, gy, actions, commands, 1, results);
+    return gridnet_step(stream, game, state, state, lanes, actions, &commands, results);
+}
+
+int nanorts_amd_gridnet_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
+                                  int64_t lanes, const int32_t* actions, const nanorts_commands* commands,
+                                  nanorts_gridnet_results results) {
+    return gridnet_step(stream, game, from, state, lanes, actions, commands, results);
 }
 
 // The seat rollout's first pass (k_seat_rollout_pair): the bot's layout on

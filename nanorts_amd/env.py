@@ -54,6 +54,9 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return t.data_ptr()
 
 
+_STATE_FIELDS = frozenset(native.STATE_FIELDS)
+
+
 # The feature-map dtypes the reference publishes
 # (src/nanorts/observations/symbolic.py:48-52), narrowest last.
 FEATURE_MAP_DTYPES: Final = (torch.int32, torch.int16, torch.uint8)
@@ -135,6 +138,11 @@ class State:
     def clone(self) -> "State":
         return State({k: v.clone() for k, v in self.leaves.items()})
 
+    def successor(self) -> "State":
+        """Uninitialised leaves like these, for a step to fill (an entry of
+        `leaves` that is no State leaf is copied)."""
+        return State({k: torch.empty_like(v) if k in _STATE_FIELDS else v.clone() for k, v in self.leaves.items()})
+
     def numpy(self) -> dict[str, np.ndarray]:
         return {k: v.cpu().numpy() for k, v in self.leaves.items()}
 
@@ -155,6 +163,31 @@ class EnvironmentState:
 
     def clone(self) -> "EnvironmentState":
         return EnvironmentState(self.core_state.clone(), self.environment_root.clone(), self.episode_index.clone())
+
+    @property
+    def is_contiguous(self) -> bool:
+        """Whether a kernel can read every leaf where it lies."""
+        leaves = self.core_state.leaves
+        return (all(leaves[name].is_contiguous() for name in native.STATE_FIELDS[:-2])
+                and self.environment_root.is_contiguous() and self.episode_index.is_contiguous())
+
+    def successor(self) -> "EnvironmentState":
+        """Uninitialised buffers like these, for a step to fill."""
+        return EnvironmentState(self.core_state.successor(), torch.empty_like(self.environment_root),
+                                torch.empty_like(self.episode_index))
+
+    def step_buffers(self, donate: bool) -> tuple["EnvironmentState", "EnvironmentState"]:
+        """(the state a step launch reads, the state it writes): this one for
+        both where the caller donates it; else this one and fresh buffers, so
+        that the step leaves it as it is without a copy before the launch.  A
+        state with a strided leaf (an expanded or sliced tensor, which the
+        kernels do not read) is copied first."""
+        if donate:
+            return self, self
+        if self.is_contiguous:
+            return self, self.successor()
+        copied = self.clone()
+        return copied, copied
 
     def native(self) -> native.State:
         leaves = self.core_state.leaves
@@ -415,7 +448,7 @@ class NanoRTS:
         return {"player": list(self.agents)}
 
     def _fused_step(self, state: EnvironmentState, actions: dict[str, torch.Tensor], donate: bool, reset: bool):
-        nxt = state if donate else state.clone()
+        before, nxt = state.step_buffers(donate)
         L = nxt.num_envs
         b = self.bucket
         acts = self._stack_actions(actions, L)
@@ -442,12 +475,10 @@ class NanoRTS:
             _ptr(out["reward"]), _ptr(out["done"]), _ptr(out["terminated"]), _ptr(out["truncated"]),
             _ptr(out["winner"]), _ptr(out["spawn_overflowed"]), _ptr(maps), _ptr(scalars), _ptr(fmaps), _ptr(fscal),
             _ptr(comps), _ptr(out["spawn_overflow"]))
-        if reset:
-            native.check(self.lib.nanorts_amd_env_step(_stream(), self.dev.ref, nxt.native(), L, _ptr(acts), self.partial,
-                                                   results), "nanorts_amd_env_step")
-        else:
-            native.check(self.lib.nanorts_amd_env_transition(_stream(), self.dev.ref, nxt.native(), L, _ptr(acts),
-                                                         self.partial, results), "nanorts_amd_env_transition")
+        written = nxt.native()
+        native.check(self.lib.nanorts_amd_env_step_from(_stream(), self.dev.ref, written if before is nxt
+                                                        else before.native(), written, L, _ptr(acts), self.partial,
+                                                        int(reset), results), "nanorts_amd_env_step_from")
         obs = self._symbolic(maps, scalars) if symbolic else self._pixels(maps, scalars)
         rewards = {agent: out["reward"][:, p] for p, agent in enumerate(self.agents)}
         dones = {agent: out["done"] for agent in self.agents} | {ALL_AGENTS: out["done"]}

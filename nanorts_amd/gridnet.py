@@ -253,19 +253,17 @@ class GridNet:
     def step(self, state: EnvironmentState, actions: torch.Tensor, *, donate: bool = False) -> GridNetStep:
         """env.step (src/nanorts/adapters/gridnet/env.py:65-70); with
         donate=True the input state's buffers are updated in place."""
-        nxt = state if donate else state.clone()
-        acts = self._actions(actions, nxt.num_envs, PLAYER_COUNT)
-        return self._step(nxt, acts, None)
+        acts = self._actions(actions, state.num_envs, PLAYER_COUNT)
+        return self._step(*state.step_buffers(donate), acts, None)
 
     def step_against(self, state: EnvironmentState, actions: torch.Tensor, commands: dict[str, torch.Tensor], *,
                      donate: bool = False) -> GridNetStep:
         """env.step_against (src/nanorts/adapters/gridnet/env.py:73-83): player 0
         plays the per-cell actions int32[L, H, W, 7], player 1 the given
         Commands ([L, 2, C] per field; player 0's rows are not read)."""
-        nxt = state if donate else state.clone()
-        acts = self._actions(actions, nxt.num_envs, 1)
+        acts = self._actions(actions, state.num_envs, 1)
         given = {f: commands[f].to(device=self.device, dtype=torch.int32).contiguous() for f in _COMMAND_FIELDS}
-        return self._step(nxt, acts, given)
+        return self._step(*state.step_buffers(donate), acts, given)
 
     # -------------------------------------------------------------- helpers
     def _actions(self, actions: torch.Tensor, L: int, players: int) -> torch.Tensor:
@@ -278,7 +276,8 @@ class GridNet:
             raise ModelError(f"gridnet actions have dtype {acts.dtype}, expected int32")
         return acts.contiguous()
 
-    def _step(self, nxt: EnvironmentState, acts: torch.Tensor, given: dict[str, torch.Tensor] | None) -> GridNetStep:
+    def _step(self, before: EnvironmentState, nxt: EnvironmentState, acts: torch.Tensor,
+              given: dict[str, torch.Tensor] | None) -> GridNetStep:
         L, d, y = nxt.num_envs, self.device, self.layout
         comps = torch.empty((L, PLAYER_COUNT, len(REWARD_COMPONENTS)), dtype=torch.float32, device=d)
         rdones = torch.empty((L, PLAYER_COUNT, len(REWARD_COMPONENTS)), dtype=torch.bool, device=d)
@@ -291,14 +290,11 @@ class GridNet:
         results = native.GridNetResults(_ptr(comps), _ptr(rdones), _ptr(flags["terminated"]), _ptr(flags["truncated"]),
                                         _ptr(flags["done"]), _ptr(winner), _ptr(flags["spawn_overflowed"]),
                                         _ptr(final), struct, _ptr(telemetry))
-        if given is None:
-            code = self.lib.nanorts_amd_gridnet_step(_stream(), self.dev.ref, nxt.native(), L, _ptr(acts), results)
-            native.check(code, "nanorts_amd_gridnet_step")
-        else:
-            c = native.Commands(*[_ptr(given[f]) for f in _COMMAND_FIELDS])
-            code = self.lib.nanorts_amd_gridnet_step_against(_stream(), self.dev.ref, nxt.native(), L, _ptr(acts), c,
-                                                         results)
-            native.check(code, "nanorts_amd_gridnet_step_against")
+        written = nxt.native()
+        c = None if given is None else ctypes.byref(native.Commands(*[_ptr(given[f]) for f in _COMMAND_FIELDS]))
+        code = self.lib.nanorts_amd_gridnet_step_from(_stream(), self.dev.ref, written if before is nxt
+                                                      else before.native(), written, L, _ptr(acts), c, results)
+        native.check(code, "nanorts_amd_gridnet_step_from")
         return GridNetStep(environment_state=nxt, observation=obs, reward_components=comps, reward_dones=rdones,
                            terminated=flags["terminated"], truncated=flags["truncated"], done=flags["done"],
                            winner=winner, telemetry={"spawn_overflow": telemetry},

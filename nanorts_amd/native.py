@@ -100,7 +100,8 @@ EXPORTS = (
     "nanorts_amd_gridnet_decode", "nanorts_amd_gridnet_observe", "nanorts_amd_gridnet_step", "nanorts_amd_gridnet_step_against",
     "nanorts_amd_gridnet_sample_actions", "nanorts_amd_step_groups_ffi", "nanorts_amd_abstraction_act_ffi",
     "nanorts_amd_astar_search_ffi", "nanorts_amd_astar_chain_ffi", "nanorts_amd_gridnet_decode_ffi",
-    "nanorts_amd_rollout_first_pass",
+    "nanorts_amd_rollout_first_pass", "nanorts_amd_env_step_from", "nanorts_amd_seat_step_from",
+    "nanorts_amd_gridnet_step_from",
 )
 
 _I64 = ctypes.c_int64
@@ -131,6 +132,7 @@ _SIGNATURES = {
     "nanorts_amd_reset_where_done": (ctypes.c_int, [_VP, _GP, State, _I64, _VP]),
     "nanorts_amd_env_step": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, _I32, EnvResults]),
     "nanorts_amd_env_transition": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, _I32, EnvResults]),
+    "nanorts_amd_env_step_from": (ctypes.c_int, [_VP, _GP, State, State, _I64, _VP, _I32, _I32, EnvResults]),
     "nanorts_amd_decode_actions": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, Commands, _VP]),
     "nanorts_amd_sample_actions": (ctypes.c_int, [_VP, _GP, _I64, _VP, _VP, _I32, _I64, _VP]),
     "nanorts_amd_rollout": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, _I32, _I32, _I32, _I64, RolloutResults]),
@@ -142,6 +144,8 @@ _SIGNATURES = {
                                             _I32, _I64, RolloutResults]),
     "nanorts_amd_seat_step_lanes": (ctypes.c_int, [_VP, _GP, State, _I64, _I32, _I32, _VP, _I32, AbstractActions, _VP,
                                                _I32, EnvResults]),
+    "nanorts_amd_seat_step_from": (ctypes.c_int, [_VP, _GP, State, State, _I64, _I32, _I32, _I32, _VP, _VP, _I32,
+                                              AbstractActions, AbstractActions, _VP, _I32, EnvResults]),
     "nanorts_amd_seat_rollout_lanes": (ctypes.c_int, [_VP, _GP, State, _I64, _I32, _I32, _VP, _I32, _VP, AbstractActions,
                                                   _VP, _I32, _I32, _I32, _I64, RolloutResults]),
     "nanorts_amd_episode_seats": (ctypes.c_int, [_VP, _VP, _VP, _I64, _VP]),
@@ -150,6 +154,7 @@ _SIGNATURES = {
     "nanorts_amd_gridnet_observe": (ctypes.c_int, [_VP, _GP, State, _I64, GridNetObs]),
     "nanorts_amd_gridnet_step": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, GridNetResults]),
     "nanorts_amd_gridnet_step_against": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, Commands, GridNetResults]),
+    "nanorts_amd_gridnet_step_from": (ctypes.c_int, [_VP, _GP, State, State, _I64, _VP, _VP, GridNetResults]),
     "nanorts_amd_gridnet_sample_actions": (ctypes.c_int, [_VP, _GP, _I64, _VP, _VP, _I32, _I64, _VP]),
     "nanorts_amd_step_groups_ffi": (ctypes.c_int, [_VP, _I32, _VP, _VP, _VP, _VP, _VP, _I32, _I32, _I32, _I32, _I32,
                                                    _I64]),

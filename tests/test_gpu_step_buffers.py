@@ -1,0 +1,171 @@
+"""A step that is not given its input state's buffers: the launch reads one
+state and writes another.  Each step surface is compared with itself on a
+donated copy (which the other tests compare with the oracle), bit for bit,
+and the input state must stay as it was.  The boards cover both row copies
+(whole vectors and by granule), both observation branches and a state with a
+strided leaf, which is copied first.  Horizons are short, so games end and
+reset inside the steps."""
+from __future__ import annotations
+
+import dataclasses
+import sys
+
+import pytest
+
+from nanorts_amd.content import map_name_to_scenario
+
+pytestmark = pytest.mark.gpu
+
+# map, games (odd counts leave the last workgroup short)
+BOARDS = (("basesWorkers8x8", 65), ("NoWhereToRun9x8", 33), ("basesWorkers16x16", 66), ("basesWorkers24x24A", 5))
+
+
+def _say(*parts):
+    print(*parts, flush=True)
+    sys.stdout.flush()
+
+
+def _tensors(value, path="out"):
+    import torch
+
+    if isinstance(value, torch.Tensor):
+        yield path, value
+    elif dataclasses.is_dataclass(value):
+        for f in dataclasses.fields(value):
+            yield from _tensors(getattr(value, f.name), f"{path}.{f.name}")
+    elif isinstance(value, dict):
+        for k, v in value.items():
+            yield from _tensors(v, f"{path}.{k}")
+    elif isinstance(value, (list, tuple)):
+        for i, v in enumerate(value):
+            yield from _tensors(v, f"{path}[{i}]")
+
+
+def _same(want, got):
+    import torch
+
+    want, got = dict(_tensors(want)), dict(_tensors(got))
+    assert want.keys() == got.keys()
+    for path, w in want.items():
+        assert torch.equal(w, got[path]), path
+
+
+def _poison():
+    """Freed memory that is not zero, for the next allocations."""
+    import torch
+
+    for size in (1 << 12, 1 << 16, 1 << 20, 1 << 22):
+        held = [torch.full((size,), 0x5A, dtype=torch.uint8, device="cuda:0") for _ in range(40)]
+        del held
+
+
+def _compare(state, step, donated):
+    """step(state) against donated(a clone), with the input kept."""
+    before = state.clone()
+    _poison()
+    got = step(state)
+    want = donated(before.clone())
+    _same(before, state)
+    _same(want, got)
+    return want
+
+
+@pytest.mark.parametrize("name,L", BOARDS)
+@pytest.mark.parametrize("strided", [False, True])
+def test_env_step_writes_fresh_buffers(name, L, strided):
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import env as envmod
+
+    _say(f"env.step into fresh buffers {name} strided={strided}")
+    game = map_name_to_scenario(name, max_cycles=36, conflict_strategy="CANCEL_ALTERNATING")
+    env = nanorts_amd.make("NanoRTS", scenario=game, partial_observability=True, reward_components=True,
+                           device="cuda:0")
+    _, state = env.reset(envmod.env_roots(3, L))
+    env.rollout(state, 30, (5, 6), record=False)
+    ends = 0
+    for t in range(8):
+        actions = env.sample_actions(env.get_avail_actions(state, form="words"), (7, 8), t)
+        if strided:
+            wide = torch.stack([state.core_state.leaves["carried_resources"]] * 2, dim=-1)
+            state.core_state.leaves["carried_resources"] = wide[..., 0]
+        fused = env.step if t % 3 else env.step_env
+        want = _compare(state, lambda s: fused(None, s, actions), lambda s: fused(None, s, actions, donate=True))
+        state = want[1]
+        ends += int(want[3]["__all__"].sum())
+    assert ends > 0
+
+
+@pytest.mark.parametrize("name,L", BOARDS[:3])
+@pytest.mark.parametrize("rule", ["player_1", "drawn"])
+def test_seat_step_writes_fresh_buffers(name, L, rule):
+    import torch
+
+    from nanorts_amd import bots
+    from nanorts_amd import env as envmod
+
+    _say(f"seat step into fresh buffers {name} {rule}")
+    game = map_name_to_scenario(name, max_cycles=36)
+    seat = bots.SeatEnv(bots.workerRushAI, scenario=game, seat=rule, device="cuda:0")
+    _, state = seat.reset(envmod.env_roots(4, L))
+    seat.rollout(state, 30, (5, 6), record=False)
+    ends = 0
+    for t in range(8):
+        words = seat.env.get_avail_actions(state.environment_state, form="words")
+        drawn = seat.env.sample_actions(words, (9, 9), t)
+        acts = {bots.LEARNER: torch.where(state.seat.reshape(-1, 1, 1) == 0, drawn["player_0"], drawn["player_1"])}
+        want = _compare(state, lambda s: seat.step(None, s, acts), lambda s: seat.step(None, s, acts, donate=True))
+        state = want[1]
+        ends += int(want[3]["__all__"].sum())
+    assert ends > 0
+
+
+@pytest.mark.parametrize("name,L", BOARDS)
+def test_gridnet_step_writes_fresh_buffers(name, L):
+    from nanorts_amd import env as envmod
+    from nanorts_amd import gridnet
+
+    _say(f"GridNet step into fresh buffers {name}")
+    game = map_name_to_scenario(name, max_cycles=6, conflict_strategy="CANCEL_RANDOM")
+    grid = gridnet.GridNet(game, gridnet.prepare(game, mask_form="packed"), device="cuda:0")
+    state, obs = grid.reset(envmod.env_roots(5, L))
+    mask, ends = obs.action_mask, 0
+    for t in range(9):
+        actions = grid.sample_actions(mask, (1, 2), t)
+        if t % 2:
+            commands = grid.decode_actions(actions, state)
+            first = actions[:, 0].contiguous()
+            want = _compare(state, lambda s: grid.step_against(s, first, commands),
+                            lambda s: grid.step_against(s, first, commands, donate=True))
+        else:
+            want = _compare(state, lambda s: grid.step(s, actions), lambda s: grid.step(s, actions, donate=True))
+        state, mask = want.environment_state, want.observation.action_mask
+        ends += int(want.done.sum())
+    assert ends > 0
+
+
+def test_step_from_entries_refuse_bad_arguments():
+    """Nothing is launched for a missing leaf of either state."""
+    import ctypes
+
+    from nanorts_amd import native
+
+    lib = native.load()
+    buf = (ctypes.c_uint8 * 64)()
+    addr = ctypes.cast(buf, ctypes.c_void_p)
+    whole = native.State(*[addr] * len(native.STATE_FIELDS))
+    rootless = native.State(*[addr] * (len(native.STATE_FIELDS) - 2), None, None)
+    game = map_name_to_scenario("basesWorkers8x8")
+    from nanorts_amd.env import DeviceGame
+    import torch
+
+    dev = DeviceGame(game, torch.device("cuda:0"))
+    for first, second in ((native.State(), whole), (whole, native.State()), (rootless, whole), (whole, rootless)):
+        assert lib.nanorts_amd_env_step_from(None, dev.ref, first, second, 1, addr, 0, 1, native.EnvResults()) == 1
+        assert lib.nanorts_amd_gridnet_step_from(None, dev.ref, first, second, 1, addr, None,
+                                                 native.GridNetResults()) == 1
+    carry = native.AbstractActions(*[addr] * len(native.ABSTRACT_FIELDS))
+    code = lib.nanorts_amd_seat_step_from(None, dev.ref, whole, whole, 1, 0, 4, 0, addr, None, 1, carry, carry, addr, 0,
+                                          native.EnvResults())
+    assert code == 1 and "seats" in lib.nanorts_amd_last_error().decode()
