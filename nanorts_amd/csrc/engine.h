@@ -1315,11 +1315,13 @@ NR_DEV int32_t live_slot_at(const KGame& g, const Env& e, int32_t i) {
 // lanes without LDS memory; the other lanes of the word send to a lane past
 // the word's ranks, and every lane keeps only what the word of its own rank
 // sent.  Every lane of the wave must be active.
+// `Two`: a lane holds two live slots, so a team holds up to 2 TW of them in its
+// lanes: the first pass of the fused rollout, with either team width.
 struct LiveLanes {
     int32_t count, slot;
-    int32_t slot2;  // half-wave teams: the (TW + lane)-th live slot, for counts up to 2 TW
+    int32_t slot2;  // Two: the (TW + lane)-th live slot, for counts up to 2 TW
 };
-template <int TW = kWave>
+template <int TW = kWave, bool Two = (TW != kWave)>
 NR_DEV LiveLanes live_lanes(const KGame& g, const Env& e, int lane) {
     LiveLanes out = {0, 0, 0};
     if constexpr (TW != kWave) {
@@ -1351,10 +1353,18 @@ NR_DEV LiveLanes live_lanes(const KGame& g, const Env& e, int lane) {
         if (m == 0ull) continue;
         const int32_t base = out.count, c = popc(m);
         out.count += c;
-        if (out.count > kWave) continue;
+        if (out.count > (Two ? 2 * kWave : kWave)) continue;
         const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, (uint32_t)base));
         const int32_t to = __builtin_amdgcn_inverse_ballot_w64(m) ? (int32_t)rank : (out.count & (kWave - 1));
+        if constexpr (Two) {
+            // ranks modulo 64: a word's at most 64 ranks fall on distinct
+            // lanes, and a lane keeps what the word of its own rank sent
+            const int32_t got2 = __builtin_amdgcn_ds_permute((to & (kWave - 1)) << 2, w * kWave + lane);
+            if (lane >= base && lane < out.count) out.slot = got2;
+            if (lane + kWave >= base && lane + kWave < out.count) out.slot2 = got2;
+            continue;
+        }
         const int32_t got = __builtin_amdgcn_ds_permute(to << 2, w * kWave + lane);
         const uint64_t upto = out.count >= kWave ? ~0ull : ((1ull << out.count) - 1ull);
         const uint64_t ranks = upto & ~((1ull << base) - 1ull);
@@ -1574,13 +1584,13 @@ NR_DEV void take_turn(const KGame& g, const Hdr& h, const Env& e, int lane, int3
 // `at_most_a_wave`: the caller guarantees at most 64 live slots, and the
 // path for more (member records in the phase union) is left out.  Returns
 // the new time.
-// A half-wave team (TW = 32) takes the slot-per-lane paths only: one live
-// slot per lane, or two (complete_two_per_lane) for 33..64; its caller
-// guarantees at most 64 live slots.
+// The first pass (`Two`) takes the slot-per-lane paths only: one live slot
+// per lane, or two (complete_two_per_lane); its caller guarantees at most
+// 2 TW live slots.
 template <int TW>
 NR_DEV int32_t complete_two_per_lane(const KGame& g, const Hdr& h, const Env& e, int lane, int32_t time,
                                      const LiveLanes& ll, const StepRecords* records);
-template <int TW = kWave>
+template <int TW = kWave, bool Two = (TW != kWave)>
 NR_DEV int32_t complete(const KGame& g, const Hdr& h, const Env& e_in, int lane, bool at_most_a_wave = false,
                         LiveLanes known = LiveLanes{-1, 0}, const StepRecords* records = nullptr) {
     const Env e = refresh<TW>(g, e_in);
@@ -1591,12 +1601,12 @@ NR_DEV int32_t complete(const KGame& g, const Hdr& h, const Env& e_in, int lane,
     // only live slots hold pending actions
     // the caller's copy when it holds one for this live set (a summary of
     // the state since which no unit spawned or died)
-    const LiveLanes ll = known.count >= 0 ? known : live_lanes<TW>(g, e, lane);
+    const LiveLanes ll = known.count >= 0 ? known : live_lanes<TW, Two>(g, e, lane);
     const int32_t nlive = ll.count;
-    if constexpr (TW != kWave) {
+    if constexpr (Two) {
         if (nlive > TW) return complete_two_per_lane<TW>(g, h, e, lane, time, ll, records);
     }
-    if (TW != kWave || at_most_a_wave || nlive <= kWave) {
+    if (Two || at_most_a_wave || nlive <= kWave) {
         // one live slot per lane: the members' retained actors stay in
         // their lanes and are ranked and read from there
         const int32_t s = lane < nlive ? ll.slot : 0;
@@ -1703,7 +1713,7 @@ NR_DEV int32_t complete(const KGame& g, const Hdr& h, const Env& e_in, int lane,
         }
         return time;
     }
-    if constexpr (TW != kWave) return time;
+    if constexpr (Two) return time;
     int32_t n = 0;
     for (int32_t base = 0; base < nlive; base += kWave) {
         const int32_t i = base + lane;
@@ -1795,7 +1805,7 @@ NR_DEV int32_t complete(const KGame& g, const Hdr& h, const Env& e_in, int lane,
     return time;
 }
 
-// complete() for a half-wave team with TW < nlive <= 2 TW live slots: lane i
+// complete() for a first pass with TW < nlive <= 2 TW live slots: lane i
 // holds live slots i and TW + i (set 0 and set 1).  Same members, same
 // order (pending order, ties by slot = by live index) as the one-per-lane
 // path.

@@ -314,7 +314,7 @@ int32_t games_per_cu(const Layout& y, int wpb, int waves_per_simd) {
 // one-wave path uses: the summary's bitmaps and lists that persist into the
 // next cycle's sampling and admission, and the summary's temporaries.  A
 // cycle that would need more (an irregular state,
-// more than 64 available units or live slots) is left to the second pass,
+// more than 64 available units or 128 live slots) is left to the second pass,
 // on the full block.  The command arrays, the request-by-request
 // admission's keys, completion's member records and the staging of the
 // non-packed observation have no place in this block and are never used
@@ -1664,12 +1664,18 @@ NR_DEV Env team_env(const KGame& g, int team) {
 // The cycles of one launch.  `Lean` is the first pass of the two-pass
 // launch (k_rollout_lean, on shape_for_lean's block): before each cycle it
 // checks that the cycle stays on the one-wave path (a regular state with at
-// most 64 available units and at most 64 live slots); at the first cycle
+// most TW available units and at most 2 TW live slots); at the first cycle
 // that does not, the game's state goes back to memory and out.progress
 // records that cycle, from which the second pass (k_rollout with `resume`,
 // on the full block) runs the rest.  Splitting a game's cycles between
 // launches this way gives the same result as one launch, as the state is
 // all a cycle carries.
+// A whole-wave team holds two live slots a lane as a half-wave team does: a
+// handed-over game's cycles run one after another at the full block's
+// latency (53 us a cycle on GardenOfWar64x64), whatever few games they are.
+// 4096 games there, 50 cycles a launch, 2 % of them past 64 live slots: the
+// second pass took as long as the first (2.63 and 2.45 ms) while the first
+// held one slot a lane.
 template <bool Lean, int TW = kWave>
 NR_DEV void rollout_cycles(const RolloutArgs& args) {
     static_assert(TW == kWave || Lean, "half-wave teams run the first pass only");
@@ -1715,7 +1721,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
     const bool fast = Lean || (g.fast_obs && ((((uintptr_t)args.out.feature_maps) & 7u) == 0));
     // the summary's counts stay in registers from one cycle into the next
     SlotSummary sm = {0, 0, 0, 0, false};
-    if (fast && fits) sm = summarize<TW>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
+    if (fast && fits) sm = summarize<TW, Lean>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
     if (!fits) sm.full = true;
     uint32_t ek0 = (uint32_t)tuni<TW>(e.sc[S_ROOT0]), ek1 = (uint32_t)tuni<TW>(e.sc[S_ROOT1]);
     fold_in(ek0, ek1, (uint32_t)tuni<TW>(e.sc[S_EPISODE]));
@@ -1744,8 +1750,8 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
         {
             // masks -> sample -> decode (get_avail_actions + harness + decode_actions)
             NR_ROLLOUT_PHASE
-            // (a half-wave team holds up to two live slots per lane)
-            if (Lean && (sm.irregular || sm.full || sm.nav > TW || sm.nlive > (TW == kWave ? kWave : 2 * TW))) {
+            // (the first pass holds up to two live slots per lane)
+            if (Lean && (sm.irregular || sm.full || sm.nav > TW || sm.nlive > 2 * TW)) {
                 stop = t;
                 break;
             }
@@ -1873,8 +1879,8 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
             // the summary's live lanes: sampling and admission spawn and
             // remove nothing
             const LiveLanes known = summary_live(sm);
-            const int32_t held = TW == kWave ? kWave : 2 * TW;  // live slots the lanes hold
-            int32_t time = complete<TW>(g, hdr, e, lane, Lean, (fast && sm.nlive <= held) ? known : LiveLanes{-1, 0, 0});
+            const int32_t held = Lean ? 2 * TW : kWave;  // live slots the lanes hold
+            int32_t time = complete<TW, Lean>(g, hdr, e, lane, Lean, (fast && sm.nlive <= held) ? known : LiveLanes{-1, 0, 0});
             Outcome oc = decide_counted<TW>(e, lane);
             nanorts_env_results r = {};
             if (rew) r.reward = rew + (int64_t)t * lanes * 2;
@@ -1908,7 +1914,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
                 // the sight bitmaps persist in the event counters' words, which
                 // the rollout does not count, when both planes fit there
                 const int32_t kept = 2 * g.H * g.seen_words <= 32 ? g.lay.b_events : -1;
-                sm = summarize<TW>(g, hdr, e, lane, a.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr, kept);
+                sm = summarize<TW, Lean>(g, hdr, e, lane, a.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr, kept);
             } else if (out.feature_maps || out.scalars) {
                 observe_both(g, hdr, e, slot, lane, a.partial != 0, out.feature_maps, out.scalars);
             }

@@ -350,8 +350,8 @@ struct SlotSummary {
     int32_t nav, nunits, nA, nlive;
     bool irregular;
     // this lane's live slot (live_lanes) for at most a wave of them in the
-    // low half, and, for half-wave teams, its second for at most two halves
-    // of them in the high half (slots are below 2^15): one register to carry
+    // low half, and, with `Two`, its second for at most 2 TW of them in the
+    // high half (slots are below 2^15): one register to carry
     // into the next cycle
     int32_t live_slots;
     // slot window (KGame::shift > 0): a unit spawned in the next cycle could
@@ -367,7 +367,7 @@ NR_DEV LiveLanes summary_live(const SlotSummary& sm) {
     return LiveLanes{sm.nlive, (int32_t)(int16_t)(sm.live_slots & 0xffff), sm.live_slots >> 16};
 }
 
-template <int TW = kWave>
+template <int TW = kWave, bool Two = (TW != kWave)>
 NR_DEV SlotSummary summarize_slots(const KGame& g, const Hdr& h, const Env& e_in, int lane, bool bitmaps = true) {
     const Env e = refresh<TW>(g, e_in);
     const Layout& y = g.lay;
@@ -396,7 +396,7 @@ NR_DEV SlotSummary summarize_slots(const KGame& g, const Hdr& h, const Env& e_in
     const int32_t time = tuni<TW>(e.sc[S_TIME]);
     const int32_t next_order = tuni<TW>(e.sc[S_NEXT_ORDER]);
     // only live slots hold units or pending actions
-    const LiveLanes ll = live_lanes<TW>(g, e, lane);
+    const LiveLanes ll = live_lanes<TW, Two>(g, e, lane);
     const int32_t nlive = ll.count;
     int32_t nav = 0, nunits = 0, nA = 0, reach0 = 0, reach1 = 0;
     // a PRODUCE issued in a cycle can complete in it (a produce time below 2,
@@ -405,10 +405,10 @@ NR_DEV SlotSummary summarize_slots(const KGame& g, const Hdr& h, const Env& e_in
     bool odd = false;
     for (int32_t base = 0; base < nlive; base += TW) {
         const int32_t i = base + lane;
-        // (a half-wave team takes up to two live slots a lane from live_lanes)
+        // (with `Two`, up to two live slots a lane from live_lanes)
         const int32_t s = i < nlive ? (nlive <= TW ? ll.slot
-                                                   : (TW != kWave && nlive <= 2 * TW ? (base == 0 ? ll.slot : ll.slot2)
-                                                                                     : live_slot_at(g, e, i)))
+                                                   : (Two && nlive <= 2 * TW ? (base == 0 ? ll.slot : ll.slot2)
+                                                                             : live_slot_at(g, e, i)))
                                     : 0;
         bool alive = false, available = false, entry = false, grows = false;
         if (i < nlive) {
@@ -700,10 +700,10 @@ NR_DEV void summarize_cells(const KGame& g, const Hdr& h, const Env& e_in, int l
 // `kept_seen` >= 0 is the LDS offset of sight bitmaps kept from the last
 // summary: they are stamped again only for a state whose units moved,
 // spawned or died since (S_VISDIRTY).
-template <int TW = kWave>
+template <int TW = kWave, bool Two = (TW != kWave)>
 NR_DEV SlotSummary summarize(const KGame& g, const Hdr& h, const Env& e, int lane, bool partial, uint8_t* maps0,
                              uint8_t* maps1, int32_t* scalars0, int32_t* scalars1, int32_t kept_seen = -1) {
-    const SlotSummary sm = summarize_slots<TW>(g, h, e, lane);
+    const SlotSummary sm = summarize_slots<TW, Two>(g, h, e, lane);
     const int32_t seen_at = kept_seen >= 0 ? kept_seen : g.lay.v_seen;
     const int32_t which = kept_seen >= 0 ? tuni<TW>(e.sc[S_VISDIRTY]) & 3 : 3;
     if (partial && maps0 && which != 0) {

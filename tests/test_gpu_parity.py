@@ -500,6 +500,39 @@ def test_pair_first_pass_holds_two_live_slots_and_two_entries_a_lane(first_pass,
     print("entries at the end:", (((pk == 1) | (pk == 4)) & (birth != -1)).sum(1).tolist(), flush=True)
 
 
+def test_lean_first_pass_holds_two_live_slots_a_lane(monkeypatch, oracle_threads):
+    """One game per wave with 57..86 live slots (22 neutral and up to 32 of each
+    player, the most the slot window holds): at most 64 in one slot a lane,
+    more in two, through the first pass to its end, or to the cycle in which a
+    player could outgrow the window.  All of them match the oracle."""
+    from oracle.oracle import Oracle
+
+    _first_pass(monkeypatch, "lean")
+    print("lean pass, two live slots a lane", flush=True)
+    game, partial = game_for("gow-alternating")
+    base = int((_packed(game, [0])["birth"][0] != -1).sum())
+    st = _packed(game, [n - base for n in (57, 63, 64, 65, 66, 72, 80, 86)])
+    st["player_resources"][:6] = 0
+    st["player_resources"][6:] = 40
+    oracle = Oracle(game)
+    assert (oracle.violations(st) == 0).all()
+    live = (st["birth"] != -1).sum(1)
+    assert live.min() == 57 and live.max() == 86
+    L, steps = live.size, 128
+    env = _env(game, partial)
+    dev = to_device(env, st)
+    got = env.rollout(dev, steps, (1, 2), record=True)
+    want = oracle.rollout(st, (1, 2), 0, steps, partial, threads=oracle_threads)
+    first = got["first_pass_cycles"].cpu().numpy()
+    print("first-pass cycles per game:", first.tolist(), flush=True)
+    assert (first[:6] == steps).any() and (first[live > 64] > 0).any()
+    np.testing.assert_array_equal(got["rewards"].cpu().numpy(), want["rewards"])
+    np.testing.assert_array_equal(got["dones"].cpu().numpy(), want["dones"].astype(bool))
+    np.testing.assert_array_equal(got["feature_maps"][0].cpu().numpy(), want["feature_maps"])
+    np.testing.assert_array_equal(got["scalars"][0].cpu().numpy(), want["scalars"])
+    assert_states_equal(st, to_host(dev), "lean pass, two live slots a lane")
+
+
 def test_crowded_env_step_per_call(oracle_threads):
     """env.step on the same crowded states, cycle by cycle, against the oracle."""
     import torch
