@@ -374,13 +374,13 @@ bool shape_for_lean(const nanorts_game* game, Shape* out, std::string* why) {
 // there, goes to the second pass.  On basesWorkers16x16 (70 slots a player)
 // that is 68 slots of 144: the block shrinks from 7.6 KB to about 4.6 KB.
 constexpr int32_t kSlotWindow = 32;
-nanorts_game windowed(const nanorts_game* game, int32_t* shift) {
+nanorts_game windowed(const nanorts_game* game, int32_t* shift, int32_t slots = kSlotWindow) {
     nanorts_game w = *game;
     *shift = 0;
-    if (game->capacity > kSlotWindow) {
-        *shift = game->capacity - kSlotWindow;
-        w.capacity = kSlotWindow;
-        w.entities = game->neutral + 2 * kSlotWindow;
+    if (game->capacity > slots) {
+        *shift = game->capacity - slots;
+        w.capacity = slots;
+        w.entities = game->neutral + 2 * slots;
     }
     return w;
 }
@@ -431,6 +431,28 @@ bool shape_for_first_pass(const nanorts_game* game, bool pair, bool any_occupanc
     int32_t shift = 0;
     const nanorts_game w = windowed(game, &shift);
     if (!(pair ? shape_for_pair(&w, out, any_occupancy, why) : shape_for_lean(&w, out, why))) return false;
+    // On boards of more than 32x32 cells most of a block is the occupancy grid
+    // and its bitmaps, and games last long enough for a player to outgrow 32
+    // slots, which sends the game's cycles one after another to the full
+    // block: there the one-game-per-wave window grows as far as as many games
+    // stay on a CU (GardenOfWar64x64: 32 -> 56 slots at 8 games per CU; 4096
+    // games x 50 cycles, where 0 to 13 games were handed over and none is now:
+    // 3.34 -> 2.27 ms).
+    // Smaller boards keep 32: their slots are most of the block, and the pair
+    // pass holds two live slots a lane, 64 in all.
+    if (!pair && game->cells > 1024) {
+        const int32_t games = games_per_cu(out->g.lay, out->wpb, kLeanWavesPerSimd);
+        for (int32_t slots = kSlotWindow + 8; shift > 0 && slots <= 2 * kSlotWindow; slots += 8) {
+            Shape wider;
+            int32_t cut = 0;
+            const nanorts_game more = windowed(game, &cut, slots);
+            if (!shape_for_lean(&more, &wider, why) ||
+                games_per_cu(wider.g.lay, wider.wpb, kLeanWavesPerSimd) < games)
+                break;
+            *out = wider;
+            shift = cut;
+        }
+    }
     out->g.shift = shift;
     if (shift > 0) out->g.nseg = 0;
     return true;

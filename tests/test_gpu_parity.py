@@ -501,23 +501,24 @@ def test_pair_first_pass_holds_two_live_slots_and_two_entries_a_lane(first_pass,
 
 
 def test_lean_first_pass_holds_two_live_slots_a_lane(monkeypatch, oracle_threads):
-    """One game per wave with 57..86 live slots (22 neutral and up to 32 of each
-    player, the most the slot window holds): at most 64 in one slot a lane,
-    more in two, through the first pass to its end, or to the cycle in which a
-    player could outgrow the window.  All of them match the oracle."""
+    """One game per wave with 57..130 live slots (22 neutral, up to 54 of each
+    player, whose window is wider than 32 slots on this board): at most 64 in
+    one slot a lane, up to 128 in two, through the first pass to its end, or to
+    the cycle in which a player could outgrow the window or the lanes.  All of
+    them match the oracle."""
     from oracle.oracle import Oracle
 
     _first_pass(monkeypatch, "lean")
     print("lean pass, two live slots a lane", flush=True)
     game, partial = game_for("gow-alternating")
     base = int((_packed(game, [0])["birth"][0] != -1).sum())
-    st = _packed(game, [n - base for n in (57, 63, 64, 65, 66, 72, 80, 86)])
+    st = _packed(game, [n - base for n in (57, 63, 64, 65, 66, 72, 80, 86, 100, 130)])
     st["player_resources"][:6] = 0
     st["player_resources"][6:] = 40
     oracle = Oracle(game)
     assert (oracle.violations(st) == 0).all()
     live = (st["birth"] != -1).sum(1)
-    assert live.min() == 57 and live.max() == 86
+    assert live.min() == 57 and live.max() == 130
     L, steps = live.size, 128
     env = _env(game, partial)
     dev = to_device(env, st)
