@@ -454,8 +454,10 @@ int nanorts_amd_rollout(void* stream, const nanorts_game* game, nanorts_state st
 
 /* Which first pass nanorts_amd_rollout runs for `game` when the caller asks
  * for the two-pass launch (results.progress set, feature maps 8-byte
- * aligned or absent): 2 two games per wave, 1 one game per wave, 0 none (one
- * pass on the full block); < 0 an error code.  Diagnostics only: it has no
+ * aligned or absent) of games that fill the device: 2 two games per wave, 1
+ * one game per wave, 0 none (one pass on the full block); < 0 an error code.
+ * A launch of few games (at most 16 per compute unit, 8 on boards below 256
+ * cells) runs 1 where this says 2.  Diagnostics only: it has no
  * counterpart in the reference, whose program has no such launch. */
 int nanorts_amd_rollout_first_pass(const nanorts_game* game);
 

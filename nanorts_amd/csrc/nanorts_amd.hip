@@ -3755,12 +3755,31 @@ int nanorts_amd_gridnet_sample_actions(void* stream, const nanorts_game* game, i
                   actions);
 }
 
+// Whether a launch has so few games that one game per wave is the faster
+// first pass: a wave of two games pays by issuing less, but each of its cycles
+// takes longer, and with few waves a SIMD it is the length of a cycle that
+// counts.  The line lies at 16 games per CU, all that one-game waves hold at
+// once, on boards whose cells give every lane of a wave four to encode, at 8
+// on smaller ones.  100 cycles, two games per wave against one: 16x16
+// 1.58 / 1.03 ms (1024 games), 1.65 / 1.14 (2048), 1.82 / 1.48 (4096),
+// 2.21 / 2.68 (8192); 24x24 2.42 / 1.57 (2048), 2.82 / 2.07 (4096); 32x32
+// 2.61 / 1.62 (2048), 2.72 / 2.07 (4096); 8x8 0.88 / 0.81 (1024), 0.91 / 0.89
+// (2048), 0.98 / 1.14 (4096).
+bool few_games(int64_t lanes, int32_t cells) {
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0)
+        return false;
+    return lanes <= (int64_t)(cells >= 4 * kWave ? 16 : 8) * cus;
+}
+
 // The rollout's first pass for a two-pass launch: 2 two games per wave
 // (`pair` shaped), 1 one game per wave (`lean`), 0 none.  Two games per wave
-// where that pays (shape_for_pair); the environment variable
-// NANORTS_AMD_FIRST_PASS set to "lean" or "pair" takes one game or two games
-// per wave whatever the board.
-static int choose_first_pass(const nanorts_game* game, const Shape& full, Shape* lean, Shape* pair) {
+// where that pays (shape_for_pair) and the launch's `lanes` games (0: a full
+// launch) are not few; the environment variable NANORTS_AMD_FIRST_PASS set to
+// "lean" or "pair" takes one game or two games per wave whatever the board
+// and the games.
+static int choose_first_pass(const nanorts_game* game, const Shape& full, int64_t lanes, Shape* lean, Shape* pair) {
     std::string why;
     if (!full.g.fast_obs || !shape_for_first_pass(game, false, false, lean, &why) ||
         games_per_cu(lean->g.lay, lean->wpb, kLeanWavesPerSimd) < games_per_cu(full.g.lay, full.wpb, 4))
@@ -3768,13 +3787,14 @@ static int choose_first_pass(const nanorts_game* game, const Shape& full, Shape*
     const char* mode = std::getenv("NANORTS_AMD_FIRST_PASS");
     const bool want_lean = mode && std::strcmp(mode, "lean") == 0;
     const bool want_pair = mode && std::strcmp(mode, "pair") == 0;
-    return !want_lean && shape_for_first_pass(game, true, want_pair, pair, &why) ? 2 : 1;
+    if (want_lean || (!want_pair && lanes > 0 && few_games(lanes, game->cells))) return 1;
+    return shape_for_first_pass(game, true, want_pair, pair, &why) ? 2 : 1;
 }
 
 int nanorts_amd_rollout_first_pass(const nanorts_game* game) {
     NR_SHAPE(game)
     Shape lean, pair;
-    return choose_first_pass(game, sh, &lean, &pair);
+    return choose_first_pass(game, sh, 0, &lean, &pair);
 }
 
 int nanorts_amd_rollout(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
@@ -3797,7 +3817,7 @@ int nanorts_amd_rollout(void* stream, const nanorts_game* game, nanorts_state st
     // games per CU as the full block.
     Shape lean, pair;
     const int first = results.progress != nullptr && (((uintptr_t)results.feature_maps) & 7u) == 0
-                          ? choose_first_pass(game, sh, &lean, &pair)
+                          ? choose_first_pass(game, sh, lanes, &lean, &pair)
                           : 0;
     const bool two_pass = first > 0, paired = first == 2;
     const int64_t games_per_block = paired ? 2 * pair.wpb : lean.wpb;

@@ -605,9 +605,10 @@ class NanoRTS:
         return {agent: actions[:, p] for p, agent in enumerate(self.agents)}
 
     def rollout_first_pass(self) -> str | None:
-        """The first pass rollout() runs on this game (with two_pass): "pair"
-        (two games per wave), "lean" (one game per wave) or None (one pass
-        on the full block).  The environment variable NANORTS_AMD_FIRST_PASS
+        """The first pass rollout() runs on this game (with two_pass) where
+        the games fill the device: "pair" (two games per wave), "lean" (one
+        game per wave, also for a rollout of few games) or None (one pass on
+        the full block).  The environment variable NANORTS_AMD_FIRST_PASS
         ("lean" or "pair") overrides the library's choice by board."""
         code = self.lib.nanorts_amd_rollout_first_pass(self.dev.ref)
         if code < 0:
