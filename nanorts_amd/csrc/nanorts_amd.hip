@@ -431,16 +431,16 @@ bool shape_for_first_pass(const nanorts_game* game, bool pair, bool any_occupanc
     int32_t shift = 0;
     const nanorts_game w = windowed(game, &shift);
     if (!(pair ? shape_for_pair(&w, out, any_occupancy, why) : shape_for_lean(&w, out, why))) return false;
-    // On boards of more than 32x32 cells most of a block is the occupancy grid
-    // and its bitmaps, and games last long enough for a player to outgrow 32
-    // slots, which sends the game's cycles one after another to the full
+    // A board laid out for 128 or more slots per player starts with many units
+    // or has room and resources for them, so its players do outgrow 32 slots,
+    // which sends the rest of a game's cycles, one after another, to the full
     // block: there the one-game-per-wave window grows as far as as many games
-    // stay on a CU (GardenOfWar64x64: 32 -> 56 slots at 8 games per CU; 4096
-    // games x 50 cycles, where 0 to 13 games were handed over and none is now:
-    // 3.34 -> 2.27 ms).
-    // Smaller boards keep 32: their slots are most of the block, and the pair
-    // pass holds two live slots a lane, 64 in all.
-    if (!pair && game->cells > 1024) {
+    // stay on a CU.  GardenOfWar64x64: 32 -> 56 slots at 8 games per CU, 4096
+    // games x 50 cycles, where 0 to 13 games were handed over and none is now,
+    // 3.34 -> 2.27 ms; FourBasesWorkers12x12: 32 -> 64 slots at 16 games, 1024
+    // games x 100 cycles, a third of them handed over, 4.07 -> 2.03 ms;
+    // TwoBasesBarracks16x16 2.98 -> 1.53 ms.
+    if (!pair && game->capacity >= 4 * kSlotWindow) {
         const int32_t games = games_per_cu(out->g.lay, out->wpb, kLeanWavesPerSimd);
         for (int32_t slots = kSlotWindow + 8; shift > 0 && slots <= 2 * kSlotWindow; slots += 8) {
             Shape wider;
