@@ -566,13 +566,17 @@ NR_DEV void summarize_visibility(const KGame& g, const Hdr& h, const Env& e_in, 
             if (v & 0x8000u) acc1 |= bits;
             else acc0 |= bits;
         }
+        // the partial rows gathered into sums of their own: past U * H lanes the
+        // shuffle wraps round to another row's lane, so no lane's partial row
+        // may take what it reads before the first H lanes have read it
+        uint32_t sum0 = acc0, sum1 = acc1;
         for (int32_t j = 1; j < U; ++j) {
-            acc0 |= (uint32_t)__shfl((int)acc0, lane + j * g.H, TW);
-            acc1 |= (uint32_t)__shfl((int)acc1, lane + j * g.H, TW);
+            sum0 |= (uint32_t)__shfl((int)acc0, lane + j * g.H, TW);
+            sum1 |= (uint32_t)__shfl((int)acc1, lane + j * g.H, TW);
         }
         if (lane < g.H) {
-            if (which & 1) seen[lane] = acc0;
-            if (which & 2) seen[plane + lane] = acc1;
+            if (which & 1) seen[lane] = sum0;
+            if (which & 2) seen[plane + lane] = sum1;
         }
         wave_sync();
         return;
