@@ -120,7 +120,10 @@ struct Layout {
 struct KGame {
     int32_t H, W, cells, N, C, E, T, O, strategy, max_cycles;
     int32_t side, radius, rank_bits, seen_words, stage_cells, sight_max;
-    int32_t fast_obs;  // 4-cell observation groups and the disk table apply
+    // 4-cell observation groups and the disk table apply: rows of whole groups
+    // (W % 4 == 0), or a board of whole groups whose rows are one bitmap word
+    // (a group may then span two rows)
+    int32_t fast_obs;
     int32_t disk_r;    // radius of the disk table: max(sight radius, attack range) <= 15
     int32_t wshift;    // log2(W) when W is a power of two, else -1
     int32_t tab[F_COUNT * 8];
@@ -485,18 +488,22 @@ NR_DEV void load_header(const KGame& g, const Hdr& h, const uint8_t* terrain, co
     for (int i = threadIdx.x; i < g.cells; i += blockDim.x) h.terrain[i] = (terrain && terrain[i]) ? 1 : 0;
     if (g.fast_obs) {
         // the walls as bitmap rows, the blocked plane every cycle starts
-        // from, packed from the terrain copy four cells per LDS read (W % 4
-        // == 0 keeps every row 4-byte aligned); every thread of the block
-        // calls this, so the barrier is safe
+        // from, packed from the terrain copy four cells per LDS read where
+        // W % 4 == 0 keeps every row 4-byte aligned, else cell by cell; every
+        // thread of the block calls this, so the barrier is safe
         __syncthreads();
         for (int i = threadIdx.x; i < g.H * g.seen_words; i += blockDim.x) {
             const int32_t row = i / g.seen_words, x0 = 32 * (i - row * g.seen_words);
             const int32_t n = g.W - x0 < 32 ? g.W - x0 : 32;
-            AS3 const uint32_t* cells = (AS3 const uint32_t*)(h.terrain + row * g.W + x0);
             uint32_t bits = 0u;
-            for (int32_t q = 0; q < (n >> 2); ++q) {
-                const uint32_t v = cells[q];  // one 0/1 byte per cell
-                bits |= ((v & 1u) | ((v >> 7) & 2u) | ((v >> 14) & 4u) | ((v >> 21) & 8u)) << (4 * q);
+            if ((g.W & 3) == 0) {
+                AS3 const uint32_t* cells = (AS3 const uint32_t*)(h.terrain + row * g.W + x0);
+                for (int32_t q = 0; q < (n >> 2); ++q) {
+                    const uint32_t v = cells[q];  // one 0/1 byte per cell
+                    bits |= ((v & 1u) | ((v >> 7) & 2u) | ((v >> 14) & 4u) | ((v >> 21) & 8u)) << (4 * q);
+                }
+            } else {
+                for (int32_t k = 0; k < n; ++k) bits |= (uint32_t)h.terrain[row * g.W + x0 + k] << k;
             }
             h.walls[i] = bits;
         }

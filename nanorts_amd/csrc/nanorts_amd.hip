@@ -161,7 +161,7 @@ bool shape_for(const nanorts_game* game, Shape* out, std::string* why, bool stag
     g.disk_r = g.sight_max;
     for (int t = 0; t < g.T; ++t)
         if (game->attack_range[t] > g.disk_r) g.disk_r = game->attack_range[t];
-    g.fast_obs = (g.W % 4 == 0 && g.disk_r <= 15) ? 1 : 0;
+    g.fast_obs = (g.W % 4 == 0 || (cells % 4 == 0 && g.W >= 4 && g.W <= 32)) && g.disk_r <= 15 ? 1 : 0;
     g.wshift = -1;
     for (int b = 0; b < 16; ++b)
         if ((1 << b) == g.W) g.wshift = b;
@@ -323,8 +323,8 @@ int32_t games_per_cu(const Layout& y, int wpb, int waves_per_simd) {
 bool shape_for_lean(const nanorts_game* game, Shape* out, std::string* why) {
     if (!shape_for(game, out, why)) return false;
     KGame& g = out->g;
-    if (!g.fast_obs) {
-        *why = "the first pass needs the packed observation (width a multiple of 4)";
+    if (!g.fast_obs || g.W % 4 != 0) {
+        *why = "the first pass needs rows of whole observation groups (width a multiple of 4)";
         return false;
     }
     Layout& y = g.lay;
@@ -1743,7 +1743,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
     const bool fast = Lean || (g.fast_obs && ((((uintptr_t)args.out.feature_maps) & 7u) == 0));
     // the summary's counts stay in registers from one cycle into the next
     SlotSummary sm = {0, 0, 0, 0, false};
-    if (fast && fits) sm = summarize<TW, Lean>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
+    if (fast && fits) sm = summarize<TW, Lean, Lean>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
     if (!fits) sm.full = true;
     uint32_t ek0 = (uint32_t)tuni<TW>(e.sc[S_ROOT0]), ek1 = (uint32_t)tuni<TW>(e.sc[S_ROOT1]);
     fold_in(ek0, ek1, (uint32_t)tuni<TW>(e.sc[S_EPISODE]));
@@ -1936,7 +1936,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
                 // the sight bitmaps persist in the event counters' words, which
                 // the rollout does not count, when both planes fit there
                 const int32_t kept = 2 * g.H * g.seen_words <= 32 ? g.lay.b_events : -1;
-                sm = summarize<TW, Lean>(g, hdr, e, lane, a.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr, kept);
+                sm = summarize<TW, Lean, Lean>(g, hdr, e, lane, a.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr, kept);
             } else if (out.feature_maps || out.scalars) {
                 observe_both(g, hdr, e, slot, lane, a.partial != 0, out.feature_maps, out.scalars);
             }
