@@ -424,10 +424,12 @@ int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_s
  * from the state `from` into the state `state`, whose leaves the call fills:
  * the input state stays as it is, which is the reference's env.step without
  * donation (src/nanorts/adapters/jaxmarl/facade.py:107-119).  Each leaf of
- * `state` is the same buffer as `from`'s or overlaps no leaf of it. */
+ * `state` is the same buffer as `from`'s or overlaps no leaf of it.  Agent p's
+ * action rows int32[C][7] of game l start at actions_p + l * action_stride (in
+ * elements), so that agents' actions are read where the caller holds them. */
 int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
-                              int64_t lanes, const int32_t* actions, int32_t partial, int32_t reset,
-                              nanorts_env_results results);
+                              int64_t lanes, const int32_t* actions0, const int32_t* actions1, int64_t action_stride,
+                              int32_t partial, int32_t reset, nanorts_env_results results);
 
 /* The JaxMARL request (src/nanorts/adapters/jaxmarl/env.py:181-184):
  * decode_actions of int32[L][2][C][7] action rows into Commands

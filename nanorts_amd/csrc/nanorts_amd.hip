@@ -1074,11 +1074,10 @@ __global__ __launch_bounds__(256) void k_reset(KGame g, int64_t lanes, nanorts_s
 // After core.step: outcome, rewards, optional final observation, auto-reset.
 // `known` / `known_time`: the cycle's outcome and time from decide_counted
 // and complete, when the caller holds them (else read from the env).
-// A half-wave team (TW = 32) writes rewards and done flags only (no event
-// counts, no final observation).
+// A half-wave team (TW = 32) writes no final observation.
 template <int TW = kWave, bool Window = false>
 NR_DEV bool finish_step(const KGame& g, const Hdr& h, const Env& e, int64_t l, int lane, bool partial,
-                        const nanorts_env_results& r, bool events, bool fast_obs = false, bool reset = true,
+                        const nanorts_env_results& r, bool events, bool reset = true,
                         const Outcome* known = nullptr, int32_t known_time = 0) {
     const bool over = known ? known->over != 0 : tuni<TW>(e.sc[S_GAME_OVER]) != 0;
     const int32_t time = known ? known_time : tuni<TW>(e.sc[S_TIME]);
@@ -1098,31 +1097,55 @@ NR_DEV bool finish_step(const KGame& g, const Hdr& h, const Env& e, int64_t l, i
             r.spawn_overflow[2 * l + 1] = e.sc[S_SO1];
         }
     }
-    if constexpr (TW == kWave) {  // the event counts and the final observation
-        if (events && r.reward_components && lane < 2) {
-            // N/adapters/rewards.py:47-71 (encode_components)
-            const AS3 int32_t* ev = at<int32_t>(e, g.lay.b_events);
-            const int p = lane, o = lane ^ 1;
-            const AS3 int32_t* prod = ev + 4 + p * 8;
-            float* out = r.reward_components + (2 * l + p) * 6;
-            out[0] = over ? (winner == p ? 1.0f : -1.0f) : 0.0f;
-            out[1] = (float)(ev[p] + ev[2 + p]);
-            out[2] = (float)prod[3];
-            out[3] = (float)(prod[1] + prod[2]);
-            out[4] = (float)(ev[20 + p * 3 + o + 1] - ev[20 + p * 3 + p + 1]);
-            out[5] = (float)(prod[4] + prod[5] + prod[6]);
-        }
-        if (fast_obs && (r.final_feature_maps || r.final_scalars)) {
-            const int64_t per = (int64_t)g.cells * 6;
-            uint8_t* m0 = r.final_feature_maps ? r.final_feature_maps + (l * 2) * per : nullptr;
-            int32_t* s0 = r.final_scalars ? r.final_scalars + l * 8 : nullptr;
-            summarize(g, h, e, lane, partial, m0, m0 ? m0 + per : nullptr, s0, s0 ? s0 + 4 : nullptr);
-        } else if (r.final_feature_maps || r.final_scalars) {
+    if (events && r.reward_components && lane < 2) {
+        // N/adapters/rewards.py:47-71 (encode_components)
+        const AS3 int32_t* ev = at<int32_t>(e, g.lay.b_events);
+        const int p = lane, o = lane ^ 1;
+        const AS3 int32_t* prod = ev + 4 + p * 8;
+        float* out = r.reward_components + (2 * l + p) * 6;
+        out[0] = over ? (winner == p ? 1.0f : -1.0f) : 0.0f;
+        out[1] = (float)(ev[p] + ev[2 + p]);
+        out[2] = (float)prod[3];
+        out[3] = (float)(prod[1] + prod[2]);
+        out[4] = (float)(ev[20 + p * 3 + o + 1] - ev[20 + p * 3 + p + 1]);
+        out[5] = (float)(prod[4] + prod[5] + prod[6]);
+    }
+    if constexpr (TW == kWave) {
+        if (r.final_feature_maps || r.final_scalars)
             observe_both(g, h, e, l, lane, partial, r.final_feature_maps, r.final_scalars);
-        }
     }
     if (done && reset) reset_env<TW, Window>(g, h, e, lane);
     return done;
+}
+
+// finish_step and the observations of the summary's encoder.  The final
+// observation is the ending state's; a game that did not end (or is not
+// reset) publishes the same one, so that it is encoded once and stored twice:
+// encoding it again made a step of 4096 games on 16x16 44.4 us instead of 40.4
+// (and of 64 games on 8x8 25.4 instead of 22.7).
+template <int TW = kWave, bool Window = false>
+NR_DEV void finish_and_show(const KGame& g, const Hdr& h, const Env& e, int64_t l, int lane, bool partial,
+                            const nanorts_env_results& r, bool events, bool reset) {
+    nanorts_env_results rest = r;
+    rest.final_feature_maps = nullptr;
+    rest.final_scalars = nullptr;
+    const bool again =
+        tuni<TW>(finish_step<TW, Window>(g, h, e, l, lane, partial, rest, events, false) && reset ? 1 : 0) != 0;
+    const int64_t maps = (int64_t)g.cells * 12;
+    // an ended game shows its ending state (when that is wanted), then the
+    // state it is reset to; the code of one pass serves both
+    int32_t ends = tuni<TW>(again && (r.final_feature_maps || r.final_scalars) ? 1 : 0);
+#pragma nounroll
+    for (;; ends = 0) {
+        if (again && ends == 0) reset_env<TW, Window>(g, h, e, lane);
+        const bool final_ = !again || ends != 0, next = ends == 0;
+        const Shown a = {final_ && r.final_feature_maps ? r.final_feature_maps + l * maps : nullptr,
+                         final_ && r.final_scalars ? r.final_scalars + l * 8 : nullptr};
+        const Shown b = {next && r.feature_maps ? r.feature_maps + l * maps : nullptr,
+                         next && r.scalars ? r.scalars + l * 8 : nullptr};
+        show_state<TW, (TW != kWave), Window>(g, h, e, lane, partial, a, b);
+        if (ends == 0) break;
+    }
 }
 
 // A step reads the state `from` and writes the state `s`: the same rows for a
@@ -1132,12 +1155,23 @@ NR_DEV bool finish_step(const KGame& g, const Hdr& h, const Env& e, int64_t l, i
 // masks-and-step turn of 64 games on 8x8 ran 207 us with the copies and
 // 130 us without, of 4096 games on 16x16 219 us and 130 us.)  A wave reads its
 // game's rows before it writes any.
+//
+// The action rows lie where the caller has them: agent p's rows of game l at
+// p's pointer + l * stride.  Agents that come as separate blocks are read from
+// them; stacking them into one tensor first read and wrote 3.9 KB a game (16x16)
+// of which the decode reads the few available units' rows.
+struct ActionRows {
+    const int32_t* agent[2];
+    int64_t stride;
+};
+NR_DEV const int32_t* action_row(const ActionRows& a, int64_t l, int32_t C, int32_t p) {
+    return p < C ? a.agent[0] + l * a.stride + p * 7 : a.agent[1] + l * a.stride + (p - C) * 7;
+}
 __global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanorts_state from, nanorts_state s,
-                           const int32_t* actions, int32_t partial, nanorts_env_results r, int32_t reset) {
+                           ActionRows actions, int32_t partial, nanorts_env_results r, int32_t reset) {
     NR_KERNEL_PROLOGUE
     load_env(g, from, l, e, LD_ALL, lane);
     count_units(g, e, lane);
-    const int32_t owned = 2 * g.C;
     uint32_t k0 = (uint32_t)uni(e.sc[S_ROOT0]), k1 = (uint32_t)uni(e.sc[S_ROOT1]);
     fold_in(k0, k1, (uint32_t)uni(e.sc[S_EPISODE]));
     const bool events = r.reward_components != nullptr;
@@ -1160,7 +1194,7 @@ __global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanort
             no_request(q);
             if (lane < n) {
                 const int32_t p = at<int16_t>(e, g.lay.a_av)[lane];
-                const int32_t* row = actions + (l * owned + p) * 7;
+                const int32_t* row = action_row(actions, l, g.C, p);
                 int32_t a[7];
 #pragma unroll
                 for (int f = 0; f < 7; ++f) a[f] = row[f];
@@ -1180,7 +1214,7 @@ __global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanort
         AS3 const int16_t* av = at<int16_t>(e, g.lay.a_av);
         for (int32_t i = lane; i < n; i += kWave) {
             const int32_t p = av[i];
-            const int32_t* row = actions + (l * owned + p) * 7;
+            const int32_t* row = action_row(actions, l, g.C, p);
             int32_t a[7];
 #pragma unroll
             for (int f = 0; f < 7; ++f) a[f] = row[f];
@@ -1189,17 +1223,14 @@ __global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanort
         wave_sync();
         env_core_step(g, hdr, e, lane, k0, k1, events, n, irregular, false);
     }
-    finish_step(g, hdr, e, l, lane, partial != 0, r, events, fast, reset != 0);
+    if (fast) {
+        finish_and_show(g, hdr, e, l, lane, partial != 0, r, events, reset != 0);
+    } else {
+        finish_step(g, hdr, e, l, lane, partial != 0, r, events, reset != 0);
+        if (r.feature_maps || r.scalars) observe_both(g, hdr, e, l, lane, partial != 0, r.feature_maps, r.scalars);
+    }
     store_env(g, s, l, e, lane);
     store_root(from, s, l, e, lane);
-    if (fast) {
-        const int64_t per = (int64_t)g.cells * 6;
-        uint8_t* m0 = r.feature_maps ? r.feature_maps + (l * 2) * per : nullptr;
-        int32_t* s0 = r.scalars ? r.scalars + l * 8 : nullptr;
-        summarize(g, hdr, e, lane, partial != 0, m0, m0 ? m0 + per : nullptr, s0, s0 ? s0 + 4 : nullptr);
-    } else if (r.feature_maps || r.scalars) {
-        observe_both(g, hdr, e, l, lane, partial != 0, r.feature_maps, r.scalars);
-    }
 }
 
 // Scripted-bot arguments: the bot region layout, the carry and the strategy.
@@ -1907,7 +1938,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
             nanorts_env_results r = {};
             if (rew) r.reward = rew + (int64_t)t * lanes * 2;
             if (dn) r.done = dn + (int64_t)t * lanes;
-            const bool done = finish_step<TW, Lean>(g, hdr, e, l, lane, a.partial != 0, r, false, false, true, &oc, time);
+            const bool done = finish_step<TW, Lean>(g, hdr, e, l, lane, a.partial != 0, r, false, true, &oc, time);
             if (done) {
                 ek0 = (uint32_t)tuni<TW>(e.sc[S_ROOT0]);
                 ek1 = (uint32_t)tuni<TW>(e.sc[S_ROOT1]);
@@ -2336,8 +2367,7 @@ NR_DEV void seat_cycles(const SeatRolloutArgs& args) {
         nanorts_env_results r = {};
         if (out.rewards) r.reward = out.rewards + tt * lanes * 2;
         if (out.dones) r.done = out.dones + tt * lanes;
-        const bool done = finish_step<TW, First>(g, hdr, refresh<TW>(g, e_in), l, lane, args.partial != 0, r, false,
-                                                 false, true, fast ? &oc : nullptr, time);
+        const bool done = finish_step<TW, First>(g, hdr, refresh<TW>(g, e_in), l, lane, args.partial != 0, r, false, true, fast ? &oc : nullptr, time);
         if (done) {
             const Env e = refresh<TW>(g, e_in);
             clear_carry_rows<TW>(g, b, ba.y, lane);
@@ -3399,30 +3429,37 @@ int nanorts_amd_reset_where_done(void* stream, const nanorts_game* game, nanorts
 // One env.step launch from the state `from` into `state` (see
 // nanorts_amd_env_step_from).
 static int env_step(void* stream, const nanorts_game* game, const nanorts_state& from, const nanorts_state& state,
-                    int64_t lanes, const int32_t* actions, int32_t partial, int32_t reset,
+                    int64_t lanes, const ActionRows& actions, int32_t partial, int32_t reset,
                     const nanorts_env_results& results, const char* call) {
     NR_SHAPE(game)
     NR_STATE(from)
     NR_STATE(state)
-    if (!actions) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
+    if (!actions.agent[0] || !actions.agent[1]) return fail(NANORTS_INVALID_ARGUMENT, "actions is NULL");
     if (!from.environment_root || !from.episode_index || !state.environment_root || !state.episode_index)
         return fail(NANORTS_INVALID_ARGUMENT, std::string(call) + " needs environment_root and episode_index");
     if (reset && !state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
     return launch(k_env_step, sh, lanes, (hipStream_t)stream, from, state, actions, partial, results, reset);
 }
+// The rows of int32[L][2][C][7] actions.
+static ActionRows stacked_rows(const nanorts_game* game, const int32_t* actions) {
+    const int64_t row = game ? (int64_t)game->capacity * 7 : 0;
+    return ActionRows{{actions, actions ? actions + row : nullptr}, 2 * row};
+}
 int nanorts_amd_env_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes, const int32_t* actions,
                      int32_t partial, nanorts_env_results results) {
-    return env_step(stream, game, state, state, lanes, actions, partial, 1, results, "env.step");
+    return env_step(stream, game, state, state, lanes, stacked_rows(game, actions), partial, 1, results, "env.step");
 }
 int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, int32_t partial, nanorts_env_results results) {
-    return env_step(stream, game, state, state, lanes, actions, partial, 0, results, "env.step_env");
+    return env_step(stream, game, state, state, lanes, stacked_rows(game, actions), partial, 0, results,
+                    "env.step_env");
 }
 int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
-                              int64_t lanes, const int32_t* actions, int32_t partial, int32_t reset,
-                              nanorts_env_results results) {
-    return env_step(stream, game, from, state, lanes, actions, partial, reset != 0, results,
-                    reset ? "env.step" : "env.step_env");
+                              int64_t lanes, const int32_t* actions0, const int32_t* actions1, int64_t action_stride,
+                              int32_t partial, int32_t reset, nanorts_env_results results) {
+    if (action_stride < 0) return fail(NANORTS_INVALID_ARGUMENT, "action_stride must be >= 0");
+    return env_step(stream, game, from, state, lanes, ActionRows{{actions0, actions1}, action_stride}, partial,
+                    reset != 0, results, reset ? "env.step" : "env.step_env");
 }
 int nanorts_amd_decode_actions(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, nanorts_command_buffers commands, uint32_t* episode_keys) {

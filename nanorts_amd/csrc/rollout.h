@@ -621,9 +621,10 @@ NR_DEV void summarize_visibility(const KGame& g, const Hdr& h, const Env& e_in, 
 // grid, ran 100 cycles of 5001 games on NoWhereToRun9x8 in 2.90 ms, this pass
 // with the slot pass's bitmaps in 2.17 ms.  `Whole`: no group spans two rows (a
 // branch on it inside the pass cost the 16x16 rollout 2 %).
+// `again0` / `again1` take the same maps when they are set.
 template <int TW, bool Whole>
 NR_DEV void summarize_cells(const KGame& g, const Hdr& h, const Env& e_in, int lane, bool partial, uint8_t* maps0,
-                            uint8_t* maps1, int32_t seen_at) {
+                            uint8_t* maps1, int32_t seen_at, uint8_t* again0 = nullptr, uint8_t* again1 = nullptr) {
     const Env e = refresh<TW>(g, e_in);
     const Layout& y = g.lay;
     const int32_t words = g.seen_words, plane = g.H * words;
@@ -685,10 +686,19 @@ NR_DEV void summarize_cells(const KGame& g, const Hdr& h, const Env& e_in, int l
                 l4[k] = shown ? v : 0u;
                 h4[k] = (shown ? kindb[k] : 0u) | terb[k];
             }
+            const uint64_t d0 = (uint64_t)l4[0] | ((uint64_t)(h4[0] | (l4[1] << 16)) << 32);
+            const uint64_t d1 = (uint64_t)((l4[1] >> 16) | (h4[1] << 16)) | ((uint64_t)l4[2] << 32);
+            const uint64_t d2 = (uint64_t)(h4[2] | (l4[3] << 16)) | ((uint64_t)((l4[3] >> 16) | (h4[3] << 16)) << 32);
             uint64_t* dst = (uint64_t*)((pl == 0 ? maps0 : maps1) + (int64_t)c0 * 6);
-            dst[0] = (uint64_t)l4[0] | ((uint64_t)(h4[0] | (l4[1] << 16)) << 32);
-            dst[1] = (uint64_t)((l4[1] >> 16) | (h4[1] << 16)) | ((uint64_t)l4[2] << 32);
-            dst[2] = (uint64_t)(h4[2] | (l4[3] << 16)) | ((uint64_t)((l4[3] >> 16) | (h4[3] << 16)) << 32);
+            dst[0] = d0;
+            dst[1] = d1;
+            dst[2] = d2;
+            if (again0) {
+                uint64_t* rep = (uint64_t*)((pl == 0 ? again0 : again1) + (int64_t)c0 * 6);
+                rep[0] = d0;
+                rep[1] = d1;
+                rep[2] = d2;
+            }
         }
     }
     wave_sync();
@@ -724,6 +734,46 @@ NR_DEV SlotSummary summarize(const KGame& g, const Hdr& h, const Env& e, int lan
         (pl == 0 ? scalars0 : scalars1)[f] = v;
     }
     return sm;
+}
+
+// Where one state's observation goes: both agents' feature maps [2][cells][6]
+// and scalars [2][4], each NULL where it is not wanted.
+struct Shown {
+    uint8_t* maps;
+    int32_t* scalars;
+};
+
+// The observation of the current state, encoded once, into `a` and `b`: the
+// slot pass without the masks' bitmaps, the sight pass and the cell pass.
+// The maps are 8-byte aligned.
+template <int TW = kWave, bool Two = (TW != kWave), bool Whole = false>
+NR_DEV void show_state(const KGame& g, const Hdr& h, const Env& e, int lane, bool partial, Shown a, Shown b) {
+    if (!a.maps) {
+        a.maps = b.maps;
+        b.maps = nullptr;
+    }
+    if (a.maps) {
+        const SlotSummary sm = summarize_slots<TW, Two>(g, h, e, lane, false);
+        if (partial) summarize_visibility<TW>(g, h, e, lane, g.lay.v_seen, 3, sm.nunits);
+        const int32_t per = g.cells * 6;
+        uint8_t* again = b.maps;
+        if (Whole || (g.W & 3) == 0)
+            summarize_cells<TW, true>(g, h, e, lane, partial, a.maps, a.maps + per, g.lay.v_seen, again,
+                                      again ? again + per : nullptr);
+        else
+            summarize_cells<TW, false>(g, h, e, lane, partial, a.maps, a.maps + per, g.lay.v_seen, again,
+                                       again ? again + per : nullptr);
+    }
+    if ((a.scalars || b.scalars) && lane < 8) {
+        const int32_t pl = lane >> 2, f = lane & 3;
+        int32_t v;
+        if (f == 0) v = e.sc[S_RES0 + pl];
+        else if (f == 1) v = e.sc[S_RES0 + (pl ^ 1)];
+        else if (f == 2) v = e.sc[S_TIME];
+        else v = e.sc[S_ALT];
+        if (a.scalars) a.scalars[lane] = v;
+        if (b.scalars) b.scalars[lane] = v;
+    }
 }
 
 // The available owned positions in slot order (the summary's list, again,

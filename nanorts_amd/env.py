@@ -451,7 +451,7 @@ class NanoRTS:
         before, nxt = state.step_buffers(donate)
         L = nxt.num_envs
         b = self.bucket
-        acts = self._stack_actions(actions, L)
+        held, stride = self._action_rows(actions, L)
         d = self.device
         out = {
             "reward": torch.empty((L, 2), dtype=torch.float32, device=d),
@@ -477,8 +477,9 @@ class NanoRTS:
             _ptr(comps), _ptr(out["spawn_overflow"]))
         written = nxt.native()
         native.check(self.lib.nanorts_amd_env_step_from(_stream(), self.dev.ref, written if before is nxt
-                                                        else before.native(), written, L, _ptr(acts), self.partial,
-                                                        int(reset), results), "nanorts_amd_env_step_from")
+                                                        else before.native(), written, L, held[0].data_ptr(),
+                                                        held[1].data_ptr(), stride, self.partial, int(reset), results),
+                     "nanorts_amd_env_step_from")
         obs = self._symbolic(maps, scalars) if symbolic else self._pixels(maps, scalars)
         rewards = {agent: out["reward"][:, p] for p, agent in enumerate(self.agents)}
         dones = {agent: out["done"] for agent in self.agents} | {ALL_AGENTS: out["done"]}
@@ -697,6 +698,22 @@ class NanoRTS:
         if a0.stride(0) != 2 * inner or a1.data_ptr() != a0.data_ptr() + inner * a0.element_size():
             return None
         return torch.as_strided(a0, (a0.shape[0], 2, *row), (2 * inner, inner, *a0.stride()[1:]))
+
+    def _action_rows(self, actions: dict[str, torch.Tensor], L: int) -> tuple[list[torch.Tensor], int]:
+        """The agents' action rows where they lie, and the elements from one
+        game's rows to the next: separate blocks and views of one stacked
+        tensor alike, as long as a game's rows are dense and both agents have
+        one stride; stacked (and checked) by _stack_actions otherwise."""
+        rows = self.layout.actions_shape
+        dense = (rows[1], 1)
+        held = [actions.get(a) for a in self.agents] if len(actions) == PLAYER_COUNT else []
+        if held and all(isinstance(t, torch.Tensor) and t.dtype == torch.int32 and t.device == self.device
+                        and tuple(t.shape) == (L, *rows) and t.stride()[1:] == dense for t in held):
+            stride = held[0].stride(0)
+            if stride == held[1].stride(0) and stride >= 0:
+                return held, stride
+        stacked = self._stack_actions(actions, L)
+        return [stacked[:, 0], stacked[:, 1]], stacked.stride(0)
 
     def _stack_actions(self, actions: dict[str, torch.Tensor], L: int) -> torch.Tensor:
         if set(actions) != set(self.agents):

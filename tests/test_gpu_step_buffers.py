@@ -97,6 +97,37 @@ def test_env_step_writes_fresh_buffers(name, L, strided):
     assert ends > 0
 
 
+@pytest.mark.parametrize("name,L", BOARDS)
+def test_env_step_reads_actions_where_they_lie(name, L):
+    """One result for every form of the same action rows: views of one tensor,
+    a block an agent, rows inside a wider tensor, one row of every game
+    (stride 0), rows that are not dense and host arrays."""
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import env as envmod
+
+    _say(f"action rows {name}")
+    game = map_name_to_scenario(name, max_cycles=40, conflict_strategy="CANCEL_RANDOM")
+    env = nanorts_amd.make("NanoRTS", scenario=game, device="cuda:0")
+    _, state = env.reset(envmod.env_roots(3, L))
+    env.rollout(state, 31, (5, 6), record=False)
+    drawn = env.sample_actions(env.get_avail_actions(state, form="words"), (7, 8), 0)
+    stacked = torch.stack([drawn[a] for a in env.agents], dim=1)
+    want = env.step(None, state, {a: stacked[:, p] for p, a in enumerate(env.agents)})
+    blocks = {a: v.clone() for a, v in drawn.items()}
+    wide = {a: torch.cat([v, v + 1], dim=1)[:, :v.shape[1]] for a, v in drawn.items()}
+    loose = {a: torch.stack([v, v], dim=-1)[..., 0] for a, v in drawn.items()}
+    mixed = {env.agents[0]: blocks[env.agents[0]], env.agents[1]: wide[env.agents[1]]}
+    host = {a: v.cpu().numpy() for a, v in drawn.items()}
+    for actions in (blocks, wide, loose, mixed, host):
+        _same(want, env.step(None, state, actions))
+    first = {a: v[:1] for a, v in drawn.items()}
+    same_everywhere = {a: v.repeat(L, 1, 1) for a, v in first.items()}
+    expanded = {a: v.expand(L, -1, -1) for a, v in first.items()}
+    _same(env.step(None, state, same_everywhere), env.step(None, state, expanded))
+
+
 @pytest.mark.parametrize("name,L", BOARDS[:3])
 @pytest.mark.parametrize("rule", ["player_1", "drawn"])
 def test_seat_step_writes_fresh_buffers(name, L, rule):
@@ -162,7 +193,7 @@ def test_step_from_entries_refuse_bad_arguments():
 
     dev = DeviceGame(game, torch.device("cuda:0"))
     for first, second in ((native.State(), whole), (whole, native.State()), (rootless, whole), (whole, rootless)):
-        assert lib.nanorts_amd_env_step_from(None, dev.ref, first, second, 1, addr, 0, 1, native.EnvResults()) == 1
+        assert lib.nanorts_amd_env_step_from(None, dev.ref, first, second, 1, addr, addr, 1, 0, 1, native.EnvResults()) == 1
         assert lib.nanorts_amd_gridnet_step_from(None, dev.ref, first, second, 1, addr, None,
                                                  native.GridNetResults()) == 1
     carry = native.AbstractActions(*[addr] * len(native.ABSTRACT_FIELDS))
