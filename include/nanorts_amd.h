@@ -426,10 +426,14 @@ int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_s
  * donation (src/nanorts/adapters/jaxmarl/facade.py:107-119).  Each leaf of
  * `state` is the same buffer as `from`'s or overlaps no leaf of it.  Agent p's
  * action rows int32[C][7] of game l start at actions_p + l * action_stride (in
- * elements), so that agents' actions are read where the caller holds them. */
+ * elements), so that agents' actions are read where the caller holds them.
+ * `taken` (int32[L] work words of the caller, or NULL) lets a call of many
+ * games run as two launches: a first pass with two games per wave, which
+ * leaves in taken[l] whether it stepped game l, and a second for the rest;
+ * the results are the same. */
 int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
                               int64_t lanes, const int32_t* actions0, const int32_t* actions1, int64_t action_stride,
-                              int32_t partial, int32_t reset, nanorts_env_results results);
+                              int32_t partial, int32_t reset, nanorts_env_results results, int32_t* taken);
 
 /* The JaxMARL request (src/nanorts/adapters/jaxmarl/env.py:181-184):
  * decode_actions of int32[L][2][C][7] action rows into Commands

@@ -580,6 +580,9 @@ enum : uint32_t {
 
 // The staged leaves: flag, State field, Env member, element type, count.
 #define NR_LEAVES(X)                                                   \
+    NR_SLOT_LEAVES(X)                                                  \
+    X(LD_ENTITY, entity_at, entity, int16_t, cells)
+#define NR_SLOT_LEAVES(X)                                              \
     X(LD_BIRTH, birth, birth, int32_t, E)                              \
     X(LD_UTYPE, unit_type, utype, int8_t, E)                           \
     X(LD_OWNER, owner, owner, int8_t, E)                               \
@@ -593,8 +596,7 @@ enum : uint32_t {
     X(LD_PPTYPE, pending_produced_type, pptype, int8_t, E)             \
     X(LD_PISSUED, pending_issued_at, pissued, int32_t, E)              \
     X(LD_PCOMPL, pending_completes_at, pcompl, int32_t, E)             \
-    X(LD_PORDER, pending_order, porder, int32_t, E)                    \
-    X(LD_ENTITY, entity_at, entity, int16_t, cells)
+    X(LD_PORDER, pending_order, porder, int32_t, E)
 
 // The per-env scalars of row l into the block's scalar leaf (lanes below
 // S_COUNT, one scalar each).
@@ -865,6 +867,23 @@ NR_DEV void store_window_rows(const KGame& g, const nanorts_state& s, int64_t l,
         s.entity_at[l * (int64_t)g.cells + c] = (int16_t)(v >= N + C ? v + sh : v);
     }
     store_scalars(s, l, e, lane);
+}
+
+// The slots outside the window, row l of `from` into row l of `s`: a first
+// pass that writes another state than it read has only the window staged.
+template <int TW>
+NR_DEV void copy_gap_rows(const KGame& g, const nanorts_state& from, const nanorts_state& s, int64_t l, int lane) {
+    const int32_t N = g.N, C = g.C, E = g.E, sh = g.shift;
+    const int64_t row = l * (int64_t)(E + 2 * sh);
+    for (int32_t i = lane; i < 2 * sh; i += TW) {
+        const int64_t at = row + (i < sh ? N + C + i : E + i);
+#define NR_GAP(flag, field, member, type, count) const type v_##member = from.field[at];
+#define NR_GAP_OUT(flag, field, member, type, count) s.field[at] = v_##member;
+        NR_SLOT_LEAVES(NR_GAP)
+        NR_SLOT_LEAVES(NR_GAP_OUT)
+#undef NR_GAP
+#undef NR_GAP_OUT
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -459,6 +459,24 @@ bool shape_for_first_pass(const nanorts_game* game, bool pair, bool any_occupanc
 }
 
 
+// Whether a launch has so few games that one game per wave is the faster
+// first pass: a wave of two games pays by issuing less, but each of its cycles
+// takes longer, and with few waves a SIMD it is the length of a cycle that
+// counts.  The line lies at 16 games per CU, all that one-game waves hold at
+// once, on boards whose cells give every lane of a wave four to encode, at 8
+// on smaller ones.  100 cycles, two games per wave against one: 16x16
+// 1.58 / 1.03 ms (1024 games), 1.65 / 1.14 (2048), 1.82 / 1.48 (4096),
+// 2.21 / 2.68 (8192); 24x24 2.42 / 1.57 (2048), 2.82 / 2.07 (4096); 32x32
+// 2.61 / 1.62 (2048), 2.72 / 2.07 (4096); 8x8 0.88 / 0.81 (1024), 0.91 / 0.89
+// (2048), 0.98 / 1.14 (4096).
+bool few_games(int64_t lanes, int32_t cells) {
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0)
+        return false;
+    return lanes <= (int64_t)(cells >= 4 * kWave ? 16 : 8) * cus;
+}
+
 // A smaller env block for the kernels that read a few leaves: `masks` holds
 // the leaves the legality rows read, the occupancy bitmaps and the staged
 // words (k_legality); otherwise the block is empty (the samplers read only
@@ -1143,7 +1161,10 @@ NR_DEV void finish_and_show(const KGame& g, const Hdr& h, const Env& e, int64_t 
                          final_ && r.final_scalars ? r.final_scalars + l * 8 : nullptr};
         const Shown b = {next && r.feature_maps ? r.feature_maps + l * maps : nullptr,
                          next && r.scalars ? r.scalars + l * 8 : nullptr};
-        show_state<TW, (TW != kWave), Window>(g, h, e, lane, partial, a, b);
+        // (the first pass's block has the sight bitmaps in the event words,
+        // read by then, where both planes fit there)
+        const int32_t seen_at = Window && 2 * g.H * g.seen_words <= 32 ? g.lay.b_events : g.lay.v_seen;
+        show_state<TW, (TW != kWave), Window>(g, h, e, lane, partial, a, b, seen_at);
         if (ends == 0) break;
     }
 }
@@ -1167,9 +1188,27 @@ struct ActionRows {
 NR_DEV const int32_t* action_row(const ActionRows& a, int64_t l, int32_t C, int32_t p) {
     return p < C ? a.agent[0] + l * a.stride + p * 7 : a.agent[1] + l * a.stride + (p - C) * 7;
 }
+// `taken` (or NULL): the games that k_env_step_pair has stepped.
 __global__ __launch_bounds__(256) void k_env_step(KGame g, int64_t lanes, nanorts_state from, nanorts_state s,
-                           ActionRows actions, int32_t partial, nanorts_env_results r, int32_t reset) {
+                           ActionRows actions, int32_t partial, nanorts_env_results r, int32_t reset,
+                           const int32_t* taken) {
+    if (taken) {
+        // a workgroup whose games are all stepped stages nothing (the vote
+        // goes through the first words of the dynamic LDS, before the header)
+        extern __shared__ __align__(16) uint8_t nr_lds[];
+        AS3 uint32_t* votes = (AS3 uint32_t*)nr_lds;
+        const int waves = (int)(blockDim.x >> 6);
+        const int64_t l0 = (int64_t)blockIdx.x * waves + (threadIdx.x >> 6);
+        const bool left = l0 < lanes && taken[l0] == 0;
+        if ((threadIdx.x & (kWave - 1)) == 0) votes[threadIdx.x >> 6] = left ? 1u : 0u;
+        __syncthreads();
+        uint32_t any = 0u;
+        for (int w = 0; w < waves; ++w) any |= votes[w];
+        __syncthreads();
+        if (any == 0u) return;
+    }
     NR_KERNEL_PROLOGUE
+    if (taken && uni(taken[l]) != 0) return;
     load_env(g, from, l, e, LD_ALL, lane);
     count_units(g, e, lane);
     uint32_t k0 = (uint32_t)uni(e.sc[S_ROOT0]), k1 = (uint32_t)uni(e.sc[S_ROOT1]);
@@ -2006,6 +2045,139 @@ __global__ __launch_bounds__(kWave * kLeanMaxGames) void k_rollout_lean(RolloutA
 // more than 32 available units or live slots.
 __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_rollout_pair(RolloutArgs args) {
     rollout_cycles<true, 32>(args);
+}
+
+// env.step of many games: the first pass of two, with two games per wave on the
+// slot window (the block and the formulation of k_rollout_pair: 4.3 KB a game
+// on 16x16 where k_env_step's full block is 9.9 KB, so twice the games are in
+// flight; and a step in place reads and writes the window's 68 of 144 slots
+// only).  A game that does not fit (a state or an initial state outside the
+// window, an irregular state, more than 32 available units or 64 live slots, a
+// spawn that could land past the window) is left untouched for k_env_step,
+// with taken[l] = 0.  65536 games on 16x16 in place: 471 us in k_env_step,
+// 375 us in both.  Few games run in k_env_step alone: with at most one
+// game per wave a SIMD the length of one step counts, not the waves in flight
+// (few_games' line; a second launch would cost 4 us more).
+struct EnvStepArgs {
+    KGame g;  // first: fresh_game() reads it at offset 0
+    int64_t lanes;
+    nanorts_state from, s;
+    ActionRows actions;
+    int32_t partial, reset;
+    int32_t elsewhere;  // some leaf of `s` is another buffer than `from`'s
+    nanorts_env_results r;
+    int32_t* taken;
+};
+typedef const __attribute__((address_space(4))) EnvStepArgs* EnvStepArgsArg;
+NR_DEV const EnvStepArgs& fresh_env_step_args() {
+    EnvStepArgsArg p = (EnvStepArgsArg)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const EnvStepArgs*)p;
+}
+__global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_env_step_pair(EnvStepArgs args) {
+    constexpr int TW = 32;
+    (void)args;
+    uint32_t k0, k1;
+    int32_t n, nA = 0, posA[2] = {0, 0}, costA[2] = {0, 0}, playerA[2] = {0, 0};
+    SlotSummary sm;
+    Reqs q;
+    no_request(q);
+    int lane, team;
+    int64_t l;
+    {
+        const EnvStepArgs& a = fresh_env_step_args();
+        const KGame& g = a.g;
+        extern __shared__ __align__(16) uint8_t nr_lds[];
+        const Hdr hdr = header_view(g);
+        load_header(g, hdr);
+        __syncthreads();
+        lane = team_lane<TW>();
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        team = 2 * wave + team_half<TW>();
+        l = (int64_t)blockIdx.x * (2 * (blockDim.x >> 6)) + team;
+        if (l >= a.lanes) return;
+        const Env e = team_env(g, team);
+        bool fits = true;
+        if (g.shift > 0) {
+            fits = load_window_rows<TW>(g, a.from, l, e, lane);
+            load_scalars(a.from, l, e, lane);
+            wave_sync();
+        } else {
+            load_env<TW>(g, a.from, l, e, LD_ALL, lane);
+        }
+        if (fits) {
+            count_units<TW>(g, e, lane);
+            sm = summarize_slots<TW>(g, hdr, e, lane, false);
+            fits = !(sm.irregular || sm.full || sm.nav > TW || sm.nlive > 2 * TW) &&
+                   admit_entries<TW>(g, hdr, e, lane, true, &nA, posA, costA, playerA, sm.nA);
+        }
+        if (!fits) {
+            if (lane == 0) a.taken[l] = 0;
+            return;
+        }
+        n = sm.nav;
+        k0 = (uint32_t)e.sc[S_ROOT0];
+        k1 = (uint32_t)e.sc[S_ROOT1];
+        fold_in(k0, k1, (uint32_t)e.sc[S_EPISODE]);
+        const bool events = a.r.reward_components != nullptr;
+        if (events) {
+            at<int32_t>(e, g.lay.b_events)[lane] = 0;
+            wave_sync();
+        }
+        if (lane < n) {
+            const int32_t p = at<int16_t>(e, g.lay.a_av)[lane];
+            const int32_t* row = p < g.C ? a.actions.agent[0] + l * a.actions.stride + p * 7
+                                         : a.actions.agent[1] + l * a.actions.stride + (p - g.C) * 7;
+            int32_t act[7];
+#pragma unroll
+            for (int f = 0; f < 7; ++f) act[f] = row[f];
+            int32_t kind, dir, ptype, target, none;
+            decode_values(g, e, p, act, &kind, &dir, &ptype, &target, &none);
+            request_of(g, hdr, e, p, kind, dir, ptype, target, none, false, events, q);
+        }
+        wave_sync();
+    }
+    {
+        const EnvStepArgs& a = fresh_env_step_args();
+        const KGame& g = a.g;
+        const Hdr hdr = header_view(g);
+        const Env e = team_env(g, team);
+        admit_resolve<TW>(g, hdr, e, lane, k0, k1, n, nA, posA, costA, playerA, q);
+    }
+    {
+        const EnvStepArgs& a = fresh_env_step_args();
+        const KGame& g = a.g;
+        const Hdr hdr = header_view(g);
+        const Env e = team_env(g, team);
+        const int32_t time = complete<TW>(g, hdr, e, lane, true, summary_live(sm));
+        const Outcome oc = decide_counted<TW>(e, lane);
+        // a game that ends takes the initial state, which has to fit the window
+        // too; nothing has been written yet
+        if (a.reset != 0 && g.shift > 0 && (oc.over != 0 || time >= g.max_cycles) && !initial_fits_window<TW>(g, lane)) {
+            if (lane == 0) a.taken[l] = 0;
+            return;
+        }
+    }
+    {
+        const EnvStepArgs& a = fresh_env_step_args();
+        const KGame& g = a.g;
+        const Hdr hdr = header_view(g);
+        const Env e = team_env(g, team);
+        finish_and_show<TW, true>(g, hdr, e, l, lane, a.partial != 0, a.r, a.r.reward_components != nullptr, a.reset != 0);
+    }
+    {
+        const EnvStepArgs& a = fresh_env_step_args();
+        const KGame& g = a.g;
+        const Env e = team_env(g, team);
+        if (g.shift > 0) {
+            store_window_rows<TW>(g, a.s, l, e, lane);
+            if (a.elsewhere != 0) copy_gap_rows<TW>(g, a.from, a.s, l, lane);
+        } else {
+            store_env<TW>(g, a.s, l, e, lane);
+        }
+        store_root(a.from, a.s, l, e, lane);
+        if (lane == 0) a.taken[l] = 1;
+    }
 }
 
 // Fused learner-vs-bot rollout: per cycle the learner's rows sampled from
@@ -3430,7 +3602,7 @@ int nanorts_amd_reset_where_done(void* stream, const nanorts_game* game, nanorts
 // nanorts_amd_env_step_from).
 static int env_step(void* stream, const nanorts_game* game, const nanorts_state& from, const nanorts_state& state,
                     int64_t lanes, const ActionRows& actions, int32_t partial, int32_t reset,
-                    const nanorts_env_results& results, const char* call) {
+                    const nanorts_env_results& results, int32_t* taken, const char* call) {
     NR_SHAPE(game)
     NR_STATE(from)
     NR_STATE(state)
@@ -3438,7 +3610,36 @@ static int env_step(void* stream, const nanorts_game* game, const nanorts_state&
     if (!from.environment_root || !from.episode_index || !state.environment_root || !state.episode_index)
         return fail(NANORTS_INVALID_ARGUMENT, std::string(call) + " needs environment_root and episode_index");
     if (reset && !state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
-    return launch(k_env_step, sh, lanes, (hipStream_t)stream, from, state, actions, partial, results, reset);
+    // Two passes where the caller gives the work words and the games are many
+    // (see k_env_step_pair); the second steps what the first left.
+    Shape pair;
+    std::string why;
+    const bool paired = taken && lanes > 0 && !few_games(lanes, game->cells) &&
+                        ((((uintptr_t)results.feature_maps) | ((uintptr_t)results.final_feature_maps)) & 7u) == 0 &&
+                        shape_for_first_pass(game, true, false, &pair, &why);
+    if (paired) {
+        EnvStepArgs args;
+        std::memset(&args, 0, sizeof(args));
+        args.g = pair.g;
+        args.lanes = lanes;
+        args.from = from;
+        args.s = state;
+        args.actions = actions;
+        args.partial = partial;
+        args.reset = reset;
+        args.r = results;
+        args.elsewhere = std::memcmp(&from, &state, sizeof(state)) != 0;
+        args.taken = taken;
+        const int64_t blocks = (lanes + 2 * pair.wpb - 1) / (2 * pair.wpb);
+        if (blocks > 0x7fffffff) return fail(NANORTS_INVALID_ARGUMENT, "too many lanes for one launch");
+        hipLaunchKernelGGL(k_env_step_pair, dim3((unsigned)blocks), dim3((unsigned)(kWave * pair.wpb)),
+                           (size_t)pair.lds, (hipStream_t)stream, args);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess)
+            return fail(NANORTS_INTERNAL, std::string("kernel launch failed: ") + hipGetErrorString(err));
+    }
+    return launch(k_env_step, sh, lanes, (hipStream_t)stream, from, state, actions, partial, results, reset,
+                  paired ? (const int32_t*)taken : nullptr);
 }
 // The rows of int32[L][2][C][7] actions.
 static ActionRows stacked_rows(const nanorts_game* game, const int32_t* actions) {
@@ -3447,19 +3648,20 @@ static ActionRows stacked_rows(const nanorts_game* game, const int32_t* actions)
 }
 int nanorts_amd_env_step(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes, const int32_t* actions,
                      int32_t partial, nanorts_env_results results) {
-    return env_step(stream, game, state, state, lanes, stacked_rows(game, actions), partial, 1, results, "env.step");
+    return env_step(stream, game, state, state, lanes, stacked_rows(game, actions), partial, 1, results, nullptr,
+                    "env.step");
 }
 int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, int32_t partial, nanorts_env_results results) {
     return env_step(stream, game, state, state, lanes, stacked_rows(game, actions), partial, 0, results,
-                    "env.step_env");
+                    nullptr, "env.step_env");
 }
 int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
                               int64_t lanes, const int32_t* actions0, const int32_t* actions1, int64_t action_stride,
-                              int32_t partial, int32_t reset, nanorts_env_results results) {
+                              int32_t partial, int32_t reset, nanorts_env_results results, int32_t* taken) {
     if (action_stride < 0) return fail(NANORTS_INVALID_ARGUMENT, "action_stride must be >= 0");
     return env_step(stream, game, from, state, lanes, ActionRows{{actions0, actions1}, action_stride}, partial,
-                    reset != 0, results, reset ? "env.step" : "env.step_env");
+                    reset != 0, results, taken, reset ? "env.step" : "env.step_env");
 }
 int nanorts_amd_decode_actions(void* stream, const nanorts_game* game, nanorts_state state, int64_t lanes,
                            const int32_t* actions, nanorts_command_buffers commands, uint32_t* episode_keys) {
@@ -3790,24 +3992,6 @@ int nanorts_amd_gridnet_sample_actions(void* stream, const nanorts_game* game, i
     }
     return launch(k_gridnet_sample, sh, lanes, (hipStream_t)stream, mask, sample_key[0], sample_key[1], step, env0,
                   actions);
-}
-
-// Whether a launch has so few games that one game per wave is the faster
-// first pass: a wave of two games pays by issuing less, but each of its cycles
-// takes longer, and with few waves a SIMD it is the length of a cycle that
-// counts.  The line lies at 16 games per CU, all that one-game waves hold at
-// once, on boards whose cells give every lane of a wave four to encode, at 8
-// on smaller ones.  100 cycles, two games per wave against one: 16x16
-// 1.58 / 1.03 ms (1024 games), 1.65 / 1.14 (2048), 1.82 / 1.48 (4096),
-// 2.21 / 2.68 (8192); 24x24 2.42 / 1.57 (2048), 2.82 / 2.07 (4096); 32x32
-// 2.61 / 1.62 (2048), 2.72 / 2.07 (4096); 8x8 0.88 / 0.81 (1024), 0.91 / 0.89
-// (2048), 0.98 / 1.14 (4096).
-bool few_games(int64_t lanes, int32_t cells) {
-    int device = 0, cus = 0;
-    if (hipGetDevice(&device) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0)
-        return false;
-    return lanes <= (int64_t)(cells >= 4 * kWave ? 16 : 8) * cus;
 }
 
 // The rollout's first pass for a two-pass launch: 2 two games per wave

@@ -745,23 +745,24 @@ struct Shown {
 
 // The observation of the current state, encoded once, into `a` and `b`: the
 // slot pass without the masks' bitmaps, the sight pass and the cell pass.
-// The maps are 8-byte aligned.
+// The maps are 8-byte aligned; `seen_at` is where the sight bitmaps go.
 template <int TW = kWave, bool Two = (TW != kWave), bool Whole = false>
-NR_DEV void show_state(const KGame& g, const Hdr& h, const Env& e, int lane, bool partial, Shown a, Shown b) {
+NR_DEV void show_state(const KGame& g, const Hdr& h, const Env& e, int lane, bool partial, Shown a, Shown b,
+                       int32_t seen_at) {
     if (!a.maps) {
         a.maps = b.maps;
         b.maps = nullptr;
     }
     if (a.maps) {
         const SlotSummary sm = summarize_slots<TW, Two>(g, h, e, lane, false);
-        if (partial) summarize_visibility<TW>(g, h, e, lane, g.lay.v_seen, 3, sm.nunits);
+        if (partial) summarize_visibility<TW>(g, h, e, lane, seen_at, 3, sm.nunits);
         const int32_t per = g.cells * 6;
         uint8_t* again = b.maps;
         if (Whole || (g.W & 3) == 0)
-            summarize_cells<TW, true>(g, h, e, lane, partial, a.maps, a.maps + per, g.lay.v_seen, again,
+            summarize_cells<TW, true>(g, h, e, lane, partial, a.maps, a.maps + per, seen_at, again,
                                       again ? again + per : nullptr);
         else
-            summarize_cells<TW, false>(g, h, e, lane, partial, a.maps, a.maps + per, g.lay.v_seen, again,
+            summarize_cells<TW, false>(g, h, e, lane, partial, a.maps, a.maps + per, seen_at, again,
                                        again ? again + per : nullptr);
     }
     if ((a.scalars || b.scalars) && lane < 8) {

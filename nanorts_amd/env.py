@@ -54,6 +54,8 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return t.data_ptr()
 
 
+# No call of so few games runs env.step as two launches.
+_FEW_GAMES: Final = 1024
 _STATE_FIELDS = frozenset(native.STATE_FIELDS)
 
 
@@ -476,9 +478,13 @@ class NanoRTS:
             _ptr(out["winner"]), _ptr(out["spawn_overflowed"]), _ptr(maps), _ptr(scalars), _ptr(fmaps), _ptr(fscal),
             _ptr(comps), _ptr(out["spawn_overflow"]))
         written = nxt.native()
+        # work words of the two-pass launch, which the library takes for more
+        # than some thousands of games only
+        taken = torch.empty(L, dtype=torch.int32, device=d) if L > _FEW_GAMES else None
         native.check(self.lib.nanorts_amd_env_step_from(_stream(), self.dev.ref, written if before is nxt
                                                         else before.native(), written, L, held[0].data_ptr(),
-                                                        held[1].data_ptr(), stride, self.partial, int(reset), results),
+                                                        held[1].data_ptr(), stride, self.partial, int(reset), results,
+                                                        _ptr(taken)),
                      "nanorts_amd_env_step_from")
         obs = self._symbolic(maps, scalars) if symbolic else self._pixels(maps, scalars)
         rewards = {agent: out["reward"][:, p] for p, agent in enumerate(self.agents)}

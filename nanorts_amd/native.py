@@ -132,7 +132,8 @@ _SIGNATURES = {
     "nanorts_amd_reset_where_done": (ctypes.c_int, [_VP, _GP, State, _I64, _VP]),
     "nanorts_amd_env_step": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, _I32, EnvResults]),
     "nanorts_amd_env_transition": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, _I32, EnvResults]),
-    "nanorts_amd_env_step_from": (ctypes.c_int, [_VP, _GP, State, State, _I64, _VP, _VP, _I64, _I32, _I32, EnvResults]),
+    "nanorts_amd_env_step_from": (ctypes.c_int, [_VP, _GP, State, State, _I64, _VP, _VP, _I64, _I32, _I32, EnvResults,
+                                             _VP]),
     "nanorts_amd_decode_actions": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, Commands, _VP]),
     "nanorts_amd_sample_actions": (ctypes.c_int, [_VP, _GP, _I64, _VP, _VP, _I32, _I64, _VP]),
     "nanorts_amd_rollout": (ctypes.c_int, [_VP, _GP, State, _I64, _VP, _I32, _I32, _I32, _I64, RolloutResults]),

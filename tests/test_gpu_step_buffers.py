@@ -128,6 +128,48 @@ def test_env_step_reads_actions_where_they_lie(name, L):
     _same(env.step(None, state, same_everywhere), env.step(None, state, expanded))
 
 
+@pytest.mark.parametrize("name,L,partial", [("basesWorkers8x8", 2051, False), ("basesWorkers16x16", 4099, True),
+                                            ("basesWorkers32x32A", 4098, True)])
+def test_env_step_of_many_games_in_two_passes(name, L, partial, monkeypatch):
+    """More games than one pass takes: the launch of two games per wave and the
+    one for the games it leaves, against the one-pass launch on the same
+    states.  Some games start crowded (more than 32 units of a player, past
+    the slot window; one at the bound), the horizon ends games inside the
+    steps, odd counts leave half a wave empty, and the input's buffers are
+    donated or not."""
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import env as envmod
+    from tests.helpers import to_device
+    from tests.test_gpu_parity import _packed
+
+    _say(f"two-pass env.step {name}")
+    game = map_name_to_scenario(name, max_cycles=44, conflict_strategy="CANCEL_RANDOM")
+    env = nanorts_amd.make("NanoRTS", scenario=game, partial_observability=partial, reward_components=True,
+                           device="cuda:0")
+    base = int((_packed(game, [0])["birth"][0] != -1).sum())
+    crowd = to_device(env, _packed(game, [n - base for n in (20, 30, 34, 35, 36, 37, 40)], alternate=False))
+    _, state = env.reset(envmod.env_roots(3, L))
+    for k, v in crowd.core_state.leaves.items():
+        state.core_state.leaves[k][:7] = v
+        state.core_state.leaves[k][-3:] = v[-3:]
+    env.rollout(state, 36, (5, 6), record=False)
+    ends = 0
+    for t in range(12):
+        actions = env.sample_actions(env.get_avail_actions(state, form="words"), (7, 8), t)
+        with monkeypatch.context() as m:
+            m.setattr(envmod, "_FEW_GAMES", 1 << 40)
+            want = env.step(None, state.clone(), actions, donate=True)
+        before = state.clone()
+        _poison()
+        _same(want, env.step(None, state, actions))
+        _same(before, state)
+        _same(want, env.step(None, state, actions, donate=True))
+        ends += int(want[3]["__all__"].sum())
+    assert ends > 0
+
+
 @pytest.mark.parametrize("name,L", BOARDS[:3])
 @pytest.mark.parametrize("rule", ["player_1", "drawn"])
 def test_seat_step_writes_fresh_buffers(name, L, rule):
@@ -193,7 +235,7 @@ def test_step_from_entries_refuse_bad_arguments():
 
     dev = DeviceGame(game, torch.device("cuda:0"))
     for first, second in ((native.State(), whole), (whole, native.State()), (rootless, whole), (whole, rootless)):
-        assert lib.nanorts_amd_env_step_from(None, dev.ref, first, second, 1, addr, addr, 1, 0, 1, native.EnvResults()) == 1
+        assert lib.nanorts_amd_env_step_from(None, dev.ref, first, second, 1, addr, addr, 1, 0, 1, native.EnvResults(), None) == 1
         assert lib.nanorts_amd_gridnet_step_from(None, dev.ref, first, second, 1, addr, None,
                                                  native.GridNetResults()) == 1
     carry = native.AbstractActions(*[addr] * len(native.ABSTRACT_FIELDS))
