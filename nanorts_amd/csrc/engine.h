@@ -599,50 +599,43 @@ enum : uint32_t {
     X(LD_PORDER, pending_order, porder, int32_t, E)
 
 // The per-env scalars of row l into the block's scalar leaf (lanes below
-// S_COUNT, one scalar each).
+// S_COUNT, one scalar each): one load through the lane's own address (a branch
+// per scalar made thirteen memory round trips' worth of issue and waits), and
+// the game-over byte, whose lane differs.
+NR_DEV const int32_t* scalar_address(const nanorts_state& s, int64_t l, int lane) {
+    const int32_t* p = nullptr;
+    p = lane == S_TIME ? s.time + l : p;
+    p = lane == S_RES0 ? s.player_resources + 2 * l : p;
+    p = lane == S_RES1 ? s.player_resources + 2 * l + 1 : p;
+    p = lane == S_NEXT_BIRTH ? s.next_birth + l : p;
+    p = lane == S_NEXT_ORDER ? s.next_pending_order + l : p;
+    p = lane == S_ALT ? s.alternating_conflict_count + l : p;
+    p = lane == S_WINNER ? s.winner + l : p;
+    p = lane == S_SO0 ? s.spawn_overflow + 2 * l : p;
+    p = lane == S_SO1 ? s.spawn_overflow + 2 * l + 1 : p;
+    if (s.environment_root) {
+        p = lane == S_ROOT0 ? (const int32_t*)s.environment_root + 2 * l : p;
+        p = lane == S_ROOT1 ? (const int32_t*)s.environment_root + 2 * l + 1 : p;
+    }
+    if (s.episode_index) p = lane == S_EPISODE ? (const int32_t*)s.episode_index + l : p;
+    return p;
+}
 NR_DEV void load_scalars(const nanorts_state& s, int64_t l, const Env& e, int lane) {
     if (lane >= S_COUNT) return;
-    int32_t v = 0;
-    switch (lane) {
-        case S_TIME: v = s.time[l]; break;
-        case S_RES0: v = s.player_resources[2 * l]; break;
-        case S_RES1: v = s.player_resources[2 * l + 1]; break;
-        case S_NEXT_BIRTH: v = s.next_birth[l]; break;
-        case S_NEXT_ORDER: v = s.next_pending_order[l]; break;
-        case S_ALT: v = s.alternating_conflict_count[l]; break;
-        case S_GAME_OVER: v = s.game_over[l] ? 1 : 0; break;
-        case S_WINNER: v = s.winner[l]; break;
-        case S_SO0: v = s.spawn_overflow[2 * l]; break;
-        case S_SO1: v = s.spawn_overflow[2 * l + 1]; break;
-        case S_ROOT0: v = s.environment_root ? (int32_t)s.environment_root[2 * l] : 0; break;
-        case S_ROOT1: v = s.environment_root ? (int32_t)s.environment_root[2 * l + 1] : 0; break;
-        case S_EPISODE: v = s.episode_index ? (int32_t)s.episode_index[l] : 0; break;
-        case S_VISDIRTY: v = 3; break;
-        default: break;
-    }
+    const int32_t* p = scalar_address(s, l, lane);
+    int32_t v = lane == S_VISDIRTY ? 3 : 0;
+    if (p) v = *p;
+    if (lane == S_GAME_OVER) v = s.game_over[l] ? 1 : 0;
     e.sc[lane] = v;
 }
 
-// The block's scalars into row l of the state.
+// The block's scalars into row l of the state (the root stays).
 NR_DEV void store_scalars(const nanorts_state& s, int64_t l, const Env& e, int lane) {
     if (lane >= S_COUNT) return;
     const int32_t v = e.sc[lane];
-    switch (lane) {
-        case S_TIME: s.time[l] = v; break;
-        case S_RES0: s.player_resources[2 * l] = v; break;
-        case S_RES1: s.player_resources[2 * l + 1] = v; break;
-        case S_NEXT_BIRTH: s.next_birth[l] = v; break;
-        case S_NEXT_ORDER: s.next_pending_order[l] = v; break;
-        case S_ALT: s.alternating_conflict_count[l] = v; break;
-        case S_GAME_OVER: s.game_over[l] = v ? 1 : 0; break;
-        case S_WINNER: s.winner[l] = v; break;
-        case S_SO0: s.spawn_overflow[2 * l] = v; break;
-        case S_SO1: s.spawn_overflow[2 * l + 1] = v; break;
-        case S_EPISODE:
-            if (s.episode_index) s.episode_index[l] = (uint32_t)v;
-            break;
-        default: break;
-    }
+    int32_t* p = (int32_t*)scalar_address(s, l, lane);
+    if (p && lane != S_ROOT0 && lane != S_ROOT1) *p = v;
+    if (lane == S_GAME_OVER) s.game_over[l] = v ? 1 : 0;
 }
 
 // The root into row l of `s`, where a step writes another state than the one
@@ -769,50 +762,68 @@ NR_DEV void store_env(const KGame& g, const nanorts_state& s, int64_t l, const E
 // glob_slot(i), and the occupancy grid's slot numbers mapped the same way.
 // A state row holds E + 2 shift slots.
 // ---------------------------------------------------------------------------
+template <int TW>
+constexpr int kWindowSets = TW == kWave ? 2 : 3;
 // Row l of `s` into the block (l = 0 with the initial state).  False when
 // the game does not fit the window: a live slot in either gap, or an
 // occupancy entry other than -1 or a slot inside the window (the block is
 // then partly written and must not run).
-template <int TW = kWave>
+template <int TW = kWave, int kSets = 1>
 NR_DEV bool load_window_rows(const KGame& g, const nanorts_state& s, int64_t l, const Env& e, int lane) {
     const int32_t N = g.N, C = g.C, E = g.E, sh = g.shift;
     const int64_t row = l * (int64_t)(E + 2 * sh);
     bool bad = false;
-    for (int32_t i = lane; i < E; i += TW) {
-        // every leaf's load first, then the LDS stores
-        const int64_t at = row + glob_slot(g, i);
-        const int32_t birth = s.birth[at], carried = s.carried_resources[at], pnone = s.pending_none_duration[at];
-        const int32_t pissued = s.pending_issued_at[at], pcompl = s.pending_completes_at[at];
-        const int32_t porder = s.pending_order[at];
-        const int16_t cell = s.cell[at], hp = s.hit_points[at], ptarget = s.pending_target_cell[at];
-        const int8_t utype = s.unit_type[at], owner = s.owner[at], pkind = s.pending_kind[at];
-        const int8_t pdir = s.pending_direction[at], pptype = s.pending_produced_type[at];
-        e.birth[i] = birth;
-        e.carried[i] = carried;
-        e.pnone[i] = pnone;
-        e.pissued[i] = pissued;
-        e.pcompl[i] = pcompl;
-        e.porder[i] = porder;
-        e.cell[i] = cell;
-        e.hp[i] = hp;
-        e.ptarget[i] = ptarget;
-        e.utype[i] = utype;
-        e.owner[i] = owner;
-        e.pkind[i] = pkind;
-        e.pdir[i] = pdir;
-        e.pptype[i] = pptype;
+    // kSets slots a lane at a time: every leaf's load of every set first, then
+    // the LDS stores, so that a kernel's first load waits on memory once for
+    // kWindowSets * TW slots (one set at a time, a step of 65536 games on 16x16,
+    // 68 slots on 32 lanes, took 360 us instead of 326 us); a reset
+    // inside a kernel, where registers are short, takes one set
+    for (int32_t base = 0; base < E; base += kSets * TW) {
+#define NR_DECLARE(flag, field, member, type, count) type v_##member[kSets];
+        NR_SLOT_LEAVES(NR_DECLARE)
+#undef NR_DECLARE
+#pragma unroll
+        for (int k = 0; k < kSets; ++k) {
+            const int32_t i = base + k * TW + lane;
+            const int64_t at = row + glob_slot(g, i < E ? i : E - 1);
+#define NR_LOAD(flag, field, member, type, count) v_##member[k] = s.field[at];
+            NR_SLOT_LEAVES(NR_LOAD)
+#undef NR_LOAD
+        }
+#pragma unroll
+        for (int k = 0; k < kSets; ++k) {
+            const int32_t i = base + k * TW + lane;
+            if (i >= E) continue;
+#define NR_STAGE(flag, field, member, type, count) e.member[i] = v_##member[k];
+            NR_SLOT_LEAVES(NR_STAGE)
+#undef NR_STAGE
+        }
     }
     // the gaps [N + C, N + C + sh) and [E + sh, E + 2 sh) hold no live slot
+#pragma unroll 4
     for (int32_t i = lane; i < 2 * sh; i += TW) {
         const int32_t gs = i < sh ? N + C + i : E + i;
         if (s.birth[row + gs] != kAbsent) bad = true;
     }
-    for (int32_t c = lane; c < g.cells; c += TW) {
-        const int32_t v = s.entity_at[l * (int64_t)g.cells + c];
-        int32_t lv = v;
-        if (v >= N + C + sh && v < E + sh) lv = v - sh;
-        else if (v < -1 || v >= N + C) bad = true;
-        e.entity[c] = (int16_t)lv;
+    // the occupancy grid, four cells a lane where its rows allow 8-byte access
+    const int16_t* grid = s.entity_at + l * (int64_t)g.cells;
+    const auto block_slot = [&](int32_t v) {
+        if (v >= N + C + sh && v < E + sh) return v - sh;
+        if (v < -1 || v >= N + C) bad = true;
+        return v;
+    };
+    if ((((uintptr_t)grid) & 7u) == 0 && (g.cells & 3) == 0) {
+#pragma unroll 2
+        for (int32_t q = lane; q < g.cells >> 2; q += TW) {
+            const uint64_t w = ((const uint64_t*)grid)[q];
+            uint64_t o = 0ull;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                o |= (uint64_t)(uint16_t)block_slot((int32_t)(int16_t)(uint16_t)(w >> (16 * k))) << (16 * k);
+            ((AS3 uint64_t*)e.entity)[q] = o;
+        }
+    } else {
+        for (int32_t c = lane; c < g.cells; c += TW) e.entity[c] = (int16_t)block_slot(grid[c]);
     }
     return tballot<TW>(bad) == 0ull;
 }
@@ -862,9 +873,23 @@ NR_DEV void store_window_rows(const KGame& g, const nanorts_state& s, int64_t l,
         s.pending_direction[at] = pdir;
         s.pending_produced_type[at] = pptype;
     }
-    for (int32_t c = lane; c < g.cells; c += TW) {
-        const int32_t v = e.entity[c];
-        s.entity_at[l * (int64_t)g.cells + c] = (int16_t)(v >= N + C ? v + sh : v);
+    int16_t* grid = s.entity_at + l * (int64_t)g.cells;
+    if ((((uintptr_t)grid) & 7u) == 0 && (g.cells & 3) == 0) {
+        for (int32_t q = lane; q < g.cells >> 2; q += TW) {
+            const uint64_t w = ((AS3 const uint64_t*)e.entity)[q];
+            uint64_t o = 0ull;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int32_t v = (int16_t)(uint16_t)(w >> (16 * k));
+                o |= (uint64_t)(uint16_t)(v >= N + C ? v + sh : v) << (16 * k);
+            }
+            ((uint64_t*)grid)[q] = o;
+        }
+    } else {
+        for (int32_t c = lane; c < g.cells; c += TW) {
+            const int32_t v = e.entity[c];
+            grid[c] = (int16_t)(v >= N + C ? v + sh : v);
+        }
     }
     store_scalars(s, l, e, lane);
 }

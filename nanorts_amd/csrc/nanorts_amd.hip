@@ -1802,7 +1802,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
     // state, which an auto-reset copies in, does not) runs no cycle here
     bool fits = true;
     if (Lean && g.shift > 0) {
-        fits = load_window_rows<TW>(g, args.s, l, e, lane) && initial_fits_window<TW>(g, lane);
+        fits = load_window_rows<TW, kWindowSets<TW>>(g, args.s, l, e, lane) && initial_fits_window<TW>(g, lane);
         load_scalars(args.s, l, e, lane);
         wave_sync();
     } else {
@@ -2099,7 +2099,7 @@ __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_env_step_pair(EnvS
         const Env e = team_env(g, team);
         bool fits = true;
         if (g.shift > 0) {
-            fits = load_window_rows<TW>(g, a.from, l, e, lane);
+            fits = load_window_rows<TW, kWindowSets<TW>>(g, a.from, l, e, lane);
             load_scalars(a.from, l, e, lane);
             wave_sync();
         } else {
@@ -2329,7 +2329,7 @@ NR_DEV void seat_cycles(const SeatRolloutArgs& args) {
     const BotArgs& ba = args.bot;
     bool fits = true;
     if (First && g.shift > 0) {
-        fits = load_window_rows<TW>(g, args.s, l, e, lane) && initial_fits_window<TW>(g, lane);
+        fits = load_window_rows<TW, kWindowSets<TW>>(g, args.s, l, e, lane) && initial_fits_window<TW>(g, lane);
         load_scalars(args.s, l, e, lane);
         wave_sync();
     } else {
@@ -2355,7 +2355,7 @@ NR_DEV void seat_cycles(const SeatRolloutArgs& args) {
     const bool fast = First || (g.fast_obs && g.seen_words == 1 && ((((uintptr_t)out.feature_maps) & 7u) == 0));
     // the summary's counts stay in registers from one cycle into the next
     SlotSummary sm = {0, 0, 0, 0, false};
-    if (fast && fits) sm = summarize<TW>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
+    if (fast && fits) sm = summarize<TW, (TW != kWave), First>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
     if (!fits) sm.full = true;
     int32_t stop = args.steps;  // first pass: the first cycle left to the second
     // Each part of a cycle rebuilds the block's row pointers from the block
@@ -2569,7 +2569,7 @@ NR_DEV void seat_cycles(const SeatRolloutArgs& args) {
             // the sight bitmaps persist in the event counters' words, which
             // the seat step does not count, when both planes fit there
             const int32_t kept_seen = 2 * g.H * g.seen_words <= 32 ? y.b_events : -1;
-            sm = summarize<TW>(g, hdr, e, lane, args.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr,
+            sm = summarize<TW, (TW != kWave), First>(g, hdr, e, lane, args.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr,
                                kept_seen);
         } else if (out.feature_maps || out.scalars) {
             if constexpr (!First) observe_both(g, hdr, e, slot, lane, args.partial != 0, out.feature_maps, out.scalars);
@@ -4249,7 +4249,7 @@ static bool seat_pair_shape(const nanorts_game* game, int32_t strategy, int32_t 
     // are int16)
     if (!bot_args(&w, out, a, strategy, trained_type, carry, &why, true)) return false;
     KGame& g = out->g;
-    if (!g.fast_obs || g.seen_words != 1) return false;
+    if (!g.fast_obs || g.W % 4 != 0 || g.seen_words != 1) return false;
     g.shift = shift;
     if (shift > 0) g.nseg = 0;
     const Layout& y = g.lay;
