@@ -1143,162 +1143,138 @@ NR_DEV int32_t order_requests(const KGame& g, const Env& e, int lane, int32_t* n
     return n;
 }
 
-// One request: N/core/admission.py:242-289 (_admit_one) with
-// reservations.resolve (N/core/reservations.py:69-111).
-NR_DEV void admit_one(const KGame& g, const Hdr& h, const Env& e, int lane, int32_t p, int32_t n_rank, uint32_t key0,
-                      uint32_t key1, bool count_events) {
-    const Layout& y = g.lay;
-    const int32_t slot = g.N + p;
-    const int32_t player = p / g.C;
-    const int32_t kind0 = uni(at<int8_t>(e, y.c_kind)[p]);
-    const int32_t dir = uni(at<int8_t>(e, y.c_dir)[p]);
-    const int32_t ptype = uni(at<int8_t>(e, y.c_ptype)[p]);
-    const int32_t target = uni(at<int16_t>(e, y.c_target)[p]);
-    const int32_t none0 = uni(at<int32_t>(e, y.c_none)[p]);
-    const int32_t time = uni(e.sc[S_TIME]);
-    const int32_t cell = uni(e.cell[slot]);
-    const int32_t unit_type = uni(e.utype[slot]);
-    const int32_t owner = uni(e.owner[slot]);
+// One request in its lane, with what _admit_one (N/core/admission.py:242-289)
+// makes of it before reservations: legality, blocking and the durations read
+// only the board, the commands and the balances, which admission leaves as
+// they are.
+struct GeneralRequest {
+    int32_t p, slot, kind, dir, ptype, target, requested, none, cost;
+};
 
-    const int32_t requested = action_duration(g, h, unit_type, kind0, none0, ptype);
-    // _none_if_illegal
-    const bool legal = uni(can_execute(g, h, e, slot, kind0, dir, target, ptype) ? 1 : 0) != 0;
-    int32_t kind = legal ? kind0 : kKindNone;
-    int32_t none = legal ? none0 : requested;
-    // _none_if_blocked
-    if (claims_position(kind)) {
-        const int32_t pos = gidx(reserved_position(g, cell, dir), g.cells);
-        if (h.terrain[pos] != 0 || e.entity[pos] != kAbsent) {
-            kind = kKindNone;
-            none = requested;
-        }
-    }
-    // _count_admitted (:406-429)
-    if (count_events && lane == 0) {
-        AS3 int32_t* ev = at<int32_t>(e, y.b_events);
-        if (kind == kKindHarvest) ev[player] += 1;
-        if (kind == kKindReturn) ev[2 + player] += 1;
-        if (kind == kKindProduce) ev[4 + player * 8 + clampi(ptype, 0, g.T - 1)] += 1;
-        if (kind == kKindAttack) {
-            const int32_t occ = e.entity[clampi(target, 0, g.cells - 1)];
-            const int32_t towner = occ == kAbsent ? kAbsent : e.owner[clampi(occ, 0, g.E - 1)];
-            if (towner + 1 >= 0 && towner + 1 < 3) ev[20 + player * 3 + towner + 1] += 1;
-        }
-    }
-    // _requested_reservation (:340-349) and resolve
-    const bool req_claims = claims_position(kind);
-    const int32_t req_cost = kind == kKindProduce ? tabv(h, F_COST, clampi(ptype, 0, g.T - 1)) : 0;
-    if (req_claims || req_cost != 0) {
-        const int32_t req_pos = reserved_position(g, cell, dir);
-        const int32_t req_player = clampi(owner, 0, 1);
-        const int32_t balance = uni(e.sc[S_RES0 + req_player]);
-        const int32_t alt = uni(e.sc[S_ALT]);
-        AS3 int16_t* rank = at<int16_t>(e, y.b_rank);
-        int32_t same_total = 0;
-        bool any_cross = false;
-        int32_t cap = kNoCap;
-        uint32_t ek0 = key0, ek1 = key1;
-        bool have_event_key = false;
-        const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-        for (int32_t base = 0; base < n_rank; base += kWave) {
-            const int32_t j = base + lane;
-            bool same = false, cross = false;
-            int32_t dur = 0, entry = 0;
-            if (j < n_rank) {
-                entry = rank[j];
-                const int32_t k = e.pkind[entry];
-                if (k != kAbsent) {
-                    const int32_t epl = clampi(e.owner[entry], 0, 1);
-                    const int32_t ept = e.pptype[entry];
-                    const int32_t ecost = k == kKindProduce ? tabv(h, F_COST, clampi(ept, 0, g.T - 1)) : 0;
-                    const bool eclaims = claims_position(k);
-                    const int32_t epos = reserved_position(g, e.cell[entry], e.pdir[entry]);
-                    const bool shared = eclaims && req_claims && epos == req_pos;
-                    const int32_t claimed = wadd(epl == req_player ? ecost : 0, req_cost);
-                    const bool over = req_cost != 0 && claimed > 0 && claimed > balance;
-                    const bool conflict = shared || over;
-                    const bool crossc = e.pissued[entry] != time;
-                    const int32_t d = action_duration(g, h, e.utype[entry], k, e.pnone[entry], ept);
-                    const int32_t packed = wadd(wmul(d, 4), (conflict && !crossc ? 2 : 0) + (conflict && crossc ? 1 : 0));
-                    dur = packed >> 2;
-                    same = ((packed >> 1) & 1) != 0;
-                    cross = (packed & 1) != 0;
-                }
+// reservations.resolve (N/core/reservations.py:69-111) of a request that
+// claims a position or costs resources, all its values wave-uniform, against
+// the entries in LDS.  True when the request becomes a NONE of `*none`.
+NR_DEV bool resolve_one(const KGame& g, const Hdr& h, const Env& e, int lane, int32_t slot, bool req_claims,
+                        int32_t req_cost, int32_t dir, int32_t requested, int32_t time, int32_t n_rank, uint32_t key0,
+                        uint32_t key1, int32_t* none) {
+    const Layout& y = g.lay;
+    const int32_t req_pos = reserved_position(g, uni(e.cell[slot]), dir);
+    const int32_t req_player = clampi(uni(e.owner[slot]), 0, 1);
+    const int32_t balance = uni(e.sc[S_RES0 + req_player]);
+    const int32_t alt = uni(e.sc[S_ALT]);
+    AS3 int16_t* rank = at<int16_t>(e, y.b_rank);
+    int32_t same_total = 0;
+    bool any_cross = false;
+    int32_t cap = kNoCap;
+    uint32_t ek0 = key0, ek1 = key1;
+    bool have_event_key = false;
+    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    for (int32_t base = 0; base < n_rank; base += kWave) {
+        const int32_t j = base + lane;
+        bool same = false, cross = false;
+        int32_t dur = 0, entry = 0;
+        if (j < n_rank) {
+            entry = rank[j];
+            const int32_t k = e.pkind[entry];
+            if (k != kAbsent) {
+                const int32_t epl = clampi(e.owner[entry], 0, 1);
+                const int32_t ept = e.pptype[entry];
+                const int32_t ecost = k == kKindProduce ? tabv(h, F_COST, clampi(ept, 0, g.T - 1)) : 0;
+                const bool eclaims = claims_position(k);
+                const int32_t epos = reserved_position(g, e.cell[entry], e.pdir[entry]);
+                const bool shared = eclaims && req_claims && epos == req_pos;
+                const int32_t claimed = wadd(epl == req_player ? ecost : 0, req_cost);
+                const bool over = req_cost != 0 && claimed > 0 && claimed > balance;
+                const bool conflict = shared || over;
+                const bool crossc = e.pissued[entry] != time;
+                const int32_t d = action_duration(g, h, e.utype[entry], k, e.pnone[entry], ept);
+                const int32_t packed = wadd(wmul(d, 4), (conflict && !crossc ? 2 : 0) + (conflict && crossc ? 1 : 0));
+                dur = packed >> 2;
+                same = ((packed >> 1) & 1) != 0;
+                cross = (packed & 1) != 0;
             }
-            const uint64_t sm = ballot(same), cm = ballot(cross);
-            if ((sm | cm) == 0ull) continue;
-            const int32_t same_before = same_total + popc(sm & below);
-            const bool cross_before = any_cross || (cm & below) != 0ull;
-            bool cancels_req = true, cancels_pend = true;
-            if (g.strategy == NANORTS_CANCEL_ALTERNATING) {
-                cancels_req = floor_mod(wadd(alt, same_before), 2) == 0;
-                cancels_pend = !cancels_req;
-            } else if (g.strategy == NANORTS_CANCEL_RANDOM) {
-                if (!have_event_key && sm != 0ull) {
-                    // _event_key (N/core/reservations.py:297-300)
-                    fold_in(ek0, ek1, (uint32_t)time);
-                    fold_in(ek0, ek1, (uint32_t)uni(e.birth[slot]));
-                    fold_in(ek0, ek1, 0u);
-                    have_event_key = true;
-                }
-                int32_t draw = 0;
-                if (same) {
-                    uint32_t d0 = ek0, d1 = ek1;
-                    fold_in(d0, d1, (uint32_t)same_before);
-                    draw = randint01(d0, d1);
-                }
-                cancels_req = draw == 0;
-                cancels_pend = !cancels_req;
-            }
-            // _settle_durations (:169-192) for this chunk
-            int32_t incl = wave_inclusive_min((same && cancels_req) ? dur : kNoCap, lane);
-            incl = imin(incl, cap);
-            int32_t excl = __shfl_up(incl, 1u, kWave);
-            if (lane == 0) excl = cap;
-            const int32_t before = cross_before ? -1 : imin(requested, excl);
-            if (same && cancels_pend) {
-                // _cancel_pending (:207-228)
-                const int32_t settled = imin(dur, before);
-                const int32_t d2 = wadd(wmul(settled, 2), 1) >> 1;
-                e.pkind[entry] = (int8_t)kKindNone;
-                e.pdir[entry] = (int8_t)kAbsent;
-                e.pnone[entry] = d2;
-                e.ptarget[entry] = (int16_t)kAbsent;
-                e.pptype[entry] = (int8_t)kAbsent;
-                e.pcompl[entry] = wadd(e.pissued[entry], d2);
-            }
-            same_total += popc(sm);
-            any_cross = any_cross || cm != 0ull;
-            cap = __shfl(incl, kWave - 1, kWave);
         }
-        if (g.strategy == NANORTS_CANCEL_ALTERNATING && lane == 0) e.sc[S_ALT] = wadd(alt, same_total);
-        if (any_cross || cap != kNoCap) {
-            kind = kKindNone;
-            none = any_cross ? -1 : imin(requested, cap);
+        const uint64_t sm = ballot(same), cm = ballot(cross);
+        if ((sm | cm) == 0ull) continue;
+        const int32_t same_before = same_total + popc(sm & below);
+        const bool cross_before = any_cross || (cm & below) != 0ull;
+        bool cancels_req = true, cancels_pend = true;
+        if (g.strategy == NANORTS_CANCEL_ALTERNATING) {
+            cancels_req = floor_mod(wadd(alt, same_before), 2) == 0;
+            cancels_pend = !cancels_req;
+        } else if (g.strategy == NANORTS_CANCEL_RANDOM) {
+            if (!have_event_key && sm != 0ull) {
+                // _event_key (N/core/reservations.py:297-300)
+                fold_in(ek0, ek1, (uint32_t)time);
+                fold_in(ek0, ek1, (uint32_t)uni(e.birth[slot]));
+                fold_in(ek0, ek1, 0u);
+                have_event_key = true;
+            }
+            int32_t draw = 0;
+            if (same) {
+                uint32_t d0 = ek0, d1 = ek1;
+                fold_in(d0, d1, (uint32_t)same_before);
+                draw = randint01(d0, d1);
+            }
+            cancels_req = draw == 0;
+            cancels_pend = !cancels_req;
         }
-        wave_sync();
+        // _settle_durations (:169-192) for this chunk
+        int32_t incl = wave_inclusive_min((same && cancels_req) ? dur : kNoCap, lane);
+        incl = imin(incl, cap);
+        int32_t excl = __shfl_up(incl, 1u, kWave);
+        if (lane == 0) excl = cap;
+        const int32_t before = cross_before ? -1 : imin(requested, excl);
+        if (same && cancels_pend) {
+            // _cancel_pending (:207-228)
+            const int32_t settled = imin(dur, before);
+            const int32_t d2 = wadd(wmul(settled, 2), 1) >> 1;
+            e.pkind[entry] = (int8_t)kKindNone;
+            e.pdir[entry] = (int8_t)kAbsent;
+            e.pnone[entry] = d2;
+            e.ptarget[entry] = (int16_t)kAbsent;
+            e.pptype[entry] = (int8_t)kAbsent;
+            e.pcompl[entry] = wadd(e.pissued[entry], d2);
+        }
+        same_total += popc(sm);
+        any_cross = any_cross || cm != 0ull;
+        cap = __shfl(incl, kWave - 1, kWave);
     }
-    // _assign_pending_action (:374-403)
-    const int32_t duration = kind == kKindNone ? none : requested;
-    if (lane == 0) {
-        const int32_t held = e.porder[slot];
-        const int32_t next_order = e.sc[S_NEXT_ORDER];
-        e.pkind[slot] = (int8_t)kind;
-        e.pdir[slot] = (int8_t)((kind == kKindMove || kind == kKindHarvest || kind == kKindReturn || kind == kKindProduce)
-                                    ? dir
-                                    : kAbsent);
-        e.pnone[slot] = kind == kKindNone ? none : 0;
-        e.ptarget[slot] = (int16_t)(kind == kKindAttack ? target : kAbsent);
-        e.pptype[slot] = (int8_t)(kind == kKindProduce ? ptype : kAbsent);
-        e.pissued[slot] = time;
-        e.pcompl[slot] = wadd(time, duration);
-        e.porder[slot] = held == kAbsent ? next_order : held;
-        if (held == kAbsent) e.sc[S_NEXT_ORDER] = wadd(next_order, 1);
+    if (g.strategy == NANORTS_CANCEL_ALTERNATING && lane == 0) e.sc[S_ALT] = wadd(alt, same_total);
+    wave_sync();
+    *none = any_cross ? -1 : imin(requested, cap);
+    return any_cross || cap != kNoCap;
+}
+
+// _assign_pending_action (N/core/admission.py:374-403) of the lanes in `mine`,
+// requests that follow one another in admission order.
+NR_DEV void assign_requests(const Env& e, const GeneralRequest& q, bool mine, int32_t time) {
+    const int32_t next_order = uni(e.sc[S_NEXT_ORDER]);
+    const bool appends = mine && e.porder[q.slot] == kAbsent;
+    const uint64_t m = ballot(appends);
+    if (mine) {
+        const int32_t k = q.kind;
+        e.pkind[q.slot] = (int8_t)k;
+        e.pdir[q.slot] = (int8_t)((claims_position(k) || k == kKindHarvest || k == kKindReturn) ? q.dir : kAbsent);
+        e.pnone[q.slot] = k == kKindNone ? q.none : 0;
+        e.ptarget[q.slot] = (int16_t)(k == kKindAttack ? q.target : kAbsent);
+        e.pptype[q.slot] = (int8_t)(k == kKindProduce ? q.ptype : kAbsent);
+        e.pissued[q.slot] = time;
+        e.pcompl[q.slot] = wadd(time, k == kKindNone ? q.none : q.requested);
+        if (appends) e.porder[q.slot] = wadd(next_order, count_below(m));
+        if (appends && count_below(m) == 0) e.sc[S_NEXT_ORDER] = wadd(next_order, popc(m));
     }
     wave_sync();
 }
 
-// admission.admit (N/core/admission.py:181-197)
+// admission.admit (N/core/admission.py:181-197).  A request's legality and
+// blocking do not depend on the ones before it, so every request has a lane,
+// and only those that claim a position or cost resources take turns: before
+// such a turn the requests ahead of it are assigned together, so that it meets
+// the entries the one-by-one order shows it.  A walk over every request (about
+// 25 a game, a chain of LDS reads each) was nearly half of a core.step on
+// arbitrary Commands: 4 x 16384 games on 16x16 731 -> 417 us, a seat step of
+// 8192 games 359 -> 336 us.
 NR_DEV void admit(const KGame& g, const Hdr& h, const Env& e, int lane, uint32_t key0, uint32_t key1,
                   bool count_events) {
     const Layout& y = g.lay;
@@ -1308,10 +1284,65 @@ NR_DEV void admit(const KGame& g, const Hdr& h, const Env& e, int lane, uint32_t
     }
     int32_t n_rank = 0;
     const int32_t n = order_requests(g, e, lane, &n_rank);
-    AS3 int16_t* order = at<int16_t>(e, y.b_order);
-    for (int32_t i = 0; i < n; ++i) {
-        const int32_t p = uni(order[i]);
-        admit_one(g, h, e, lane, p, n_rank, key0, key1, count_events);
+    const int32_t time = uni(e.sc[S_TIME]);
+    for (int32_t base = 0; base < n; base += kWave) {
+        const int32_t m = imin(n - base, kWave);
+        const bool valid = lane < m;
+        GeneralRequest q;
+        q.p = valid ? at<int16_t>(e, y.b_order)[base + lane] : 0;
+        q.slot = g.N + q.p;
+        q.kind = valid ? at<int8_t>(e, y.c_kind)[q.p] : kKindNone;
+        q.dir = at<int8_t>(e, y.c_dir)[q.p];
+        q.ptype = at<int8_t>(e, y.c_ptype)[q.p];
+        q.target = at<int16_t>(e, y.c_target)[q.p];
+        q.none = at<int32_t>(e, y.c_none)[q.p];
+        q.requested = action_duration(g, h, e.utype[q.slot], q.kind, q.none, q.ptype);
+        // _none_if_illegal, then _none_if_blocked
+        bool waits = !valid || !can_execute(g, h, e, q.slot, q.kind, q.dir, q.target, q.ptype);
+        if (!waits && claims_position(q.kind)) {
+            const int32_t pos = gidx(reserved_position(g, e.cell[q.slot], q.dir), g.cells);
+            waits = h.terrain[pos] != 0 || e.entity[pos] != kAbsent;
+        }
+        if (waits) {
+            q.kind = kKindNone;
+            q.none = q.requested;
+        }
+        // _count_admitted (:406-429)
+        if (count_events && valid) {
+            AS3 int32_t* ev = at<int32_t>(e, y.b_events);
+            const int32_t player = q.p >= g.C ? 1 : 0;
+            int32_t counter = -1;
+            if (q.kind == kKindHarvest) counter = player;
+            if (q.kind == kKindReturn) counter = 2 + player;
+            if (q.kind == kKindProduce) counter = 4 + player * 8 + clampi(q.ptype, 0, g.T - 1);
+            if (q.kind == kKindAttack) {
+                const int32_t occ = e.entity[clampi(q.target, 0, g.cells - 1)];
+                const int32_t towner = occ == kAbsent ? kAbsent : e.owner[clampi(occ, 0, g.E - 1)];
+                if (towner + 1 >= 0 && towner + 1 < 3) counter = 20 + player * 3 + towner + 1;
+            }
+            if (counter >= 0) __atomic_fetch_add(&ev[counter], 1, __ATOMIC_RELAXED);
+        }
+        // _requested_reservation (:340-349)
+        q.cost = q.kind == kKindProduce ? tabv(h, F_COST, clampi(q.ptype, 0, g.T - 1)) : 0;
+        uint64_t turns = ballot(valid && (claims_position(q.kind) || q.cost != 0));
+        int32_t from = 0;  // the lanes below are assigned
+        while (turns != 0ull) {
+            const int32_t j = __builtin_ctzll(turns);
+            turns &= turns - 1ull;
+            if (j > from) assign_requests(e, q, lane >= from && lane < j, time);
+            from = j;
+            int32_t none = 0;
+            const bool becomes_none =
+                resolve_one(g, h, e, lane, __builtin_amdgcn_readlane(q.slot, j),
+                            claims_position(__builtin_amdgcn_readlane(q.kind, j)),
+                            __builtin_amdgcn_readlane(q.cost, j), __builtin_amdgcn_readlane(q.dir, j),
+                            __builtin_amdgcn_readlane(q.requested, j), time, n_rank, key0, key1, &none);
+            if (becomes_none && lane == j) {
+                q.kind = kKindNone;
+                q.none = none;
+            }
+        }
+        assign_requests(e, q, lane >= from && valid, time);
     }
 }
 

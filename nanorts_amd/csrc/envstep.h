@@ -384,10 +384,7 @@ NR_DEV void env_core_step(const KGame& g, const Hdr& h, const Env& e, int lane, 
         wave_sync();
     }
     if (!admit_env(g, h, e, lane, key0, key1, count_events, n, irregular, known_legal)) {
-        int32_t n_rank = 0;
-        const int32_t issued = order_requests(g, e, lane, &n_rank);
-        AS3 int16_t* order = at<int16_t>(e, g.lay.b_order);
-        for (int32_t i = 0; i < issued; ++i) admit_one(g, h, e, lane, uni(order[i]), n_rank, key0, key1, count_events);
+        admit(g, h, e, lane, key0, key1, count_events);
     }
     complete(g, h, e, lane);
     decide_counted(e, lane);

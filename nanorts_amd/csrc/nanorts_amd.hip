@@ -1985,10 +1985,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
                 if (fused) stage_requests(g, e, lane, n, q);
                 if (fast) mark_unavailable(g, e, lane);
                 ++general;
-                int32_t n_rank = 0;
-                const int32_t issued = order_requests(g, e, lane, &n_rank);
-                AS3 int16_t* order = at<int16_t>(e, g.lay.b_order);
-                for (int32_t i = 0; i < issued; ++i) admit_one(g, hdr, e, lane, uni(order[i]), n_rank, ek0, ek1, false);
+                admit(g, hdr, e, lane, ek0, ek1, false);
             }
         }
         {

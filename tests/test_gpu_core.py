@@ -71,3 +71,45 @@ def test_core_functions_match_oracle(case, oracle_threads):
                         "core.step")
     np.testing.assert_array_equal(out["reward"].cpu().numpy(), want["reward"])
     np.testing.assert_array_equal(out["admitted_produce"].cpu().numpy(), want["admitted_produce"])
+
+
+@pytest.mark.parametrize("strategy", ["CANCEL_BOTH", "CANCEL_RANDOM", "CANCEL_ALTERNATING"])
+@pytest.mark.parametrize("units", [(3, 1), (40, 24), (72, 12)], ids=["few", "one-wave", "two-waves"])
+def test_arbitrary_commands_on_crowded_boards(strategy, units, oracle_threads):
+    """core.step on Commands of any kind, legal or not, for every unit: mostly
+    moves and productions in one corner of the board, so that requests contest
+    positions and resources, units with pending actions are commanded again
+    and waiting requests stand between claiming ones; up to more requests than
+    a wave has lanes."""
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import core
+    from oracle.oracle import Oracle
+    from tests.test_gpu_parity import _crowded
+
+    print(f"arbitrary commands {strategy} {units}", flush=True)
+    torch.cuda.set_device(0)
+    game = nanorts_amd.map_name_to_scenario("GardenOfWar64x64", conflict_strategy=strategy, max_cycles=2000,
+                                            capacity_profile=False)
+    L, b = 12, game.bucket
+    st = _crowded(game, L, *units, seed=8)
+    st["player_resources"][:] = 3
+    oracle, state = Oracle(game), _core_state(st)
+    rng = np.random.default_rng(sum(units))
+    shape = (L, 2, b.per_player_capacity)
+    for t in range(10):
+        cmds = {"kind": rng.choice([-1, 0, 1, 1, 1, 2, 3, 4, 4, 5, 6], size=shape),
+                "direction": rng.integers(-1, 5, size=shape), "none_duration": rng.integers(1, 6, size=shape),
+                "target_cell": rng.integers(-1, b.cell_count + 1, size=shape),
+                "produced_type": rng.integers(-1, b.unit_type_capacity + 1, size=shape),
+                "request_order": rng.integers(-1, 2 * b.per_player_capacity, size=shape)}
+        cmds = {f: cmds[f].astype(np.int32) for f in FIELDS}
+        keys = rng.integers(0, 2**32, size=(L, 2), dtype=np.uint64).astype(np.uint32)
+        out = core.step(keys, state, {f: torch.as_tensor(cmds[f], device="cuda:0") for f in FIELDS}, game)
+        want = oracle.core_step(st, cmds, keys)
+        got = {name: leaf.cpu().numpy() for name, leaf in state.leaves.items()}
+        assert_states_equal(st, {**got, "environment_root": st["environment_root"],
+                                 "episode_index": st["episode_index"]}, f"step {t}")
+        for name in ("reward", "admitted_harvest", "admitted_return", "admitted_produce", "admitted_attack"):
+            np.testing.assert_array_equal(out[name].cpu().numpy(), want[name], err_msg=f"{name}, step {t}")
