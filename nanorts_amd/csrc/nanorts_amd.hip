@@ -588,8 +588,6 @@ bool shape_for_bots(const nanorts_game* game, Shape* out, BotLayout* by, std::st
     by->u_lkey = take(4 * C);
     by->m_claimed = take(4 * words);
     by->m_free = take(4 * words);
-    by->m_used = take(4 * words);
-    by->m_kept = take(4 * words);
     // dead once the walk starts (ranks, nearest enemies, roles, the queue's
     // scratch list, the candidate lists, the build reservations): the walk's
     // search scratch lies over them.  Enemies and own stockpiles are units of

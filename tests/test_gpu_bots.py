@@ -246,3 +246,48 @@ def test_seat_two_pass_hands_games_to_the_second_pass(bot):
     assert_states_equal(st, to_host(sst.environment_state), "final state")
     _assert_carry_equal(carry, _carry_to_host(sst.carry), "final carry")
     np.testing.assert_array_equal(got["feature_maps"][0].cpu().numpy(), want["feature_maps"])
+
+
+@pytest.mark.parametrize("name", ["basesWorkers8x8", "NoWhereToRun9x8", "FourBasesWorkers12x12", "basesWorkers16x16",
+                                  "basesWorkers32x32A", "GardenOfWar64x64"])
+def test_searches_on_crowded_boards(name):
+    """Acts and fused seat cycles from boards where up to three quarters of
+    the open cells hold a unit: straight paths that meet dead ends, paths that
+    a unit ahead in the queue closes, goals other units enclose (the flood's
+    answer, on boards of rows that are a part of a word, a word and two
+    words), more queued units than a team has lanes."""
+    import torch
+
+    from nanorts_amd import bots
+    from nanorts_amd.bots import SeatState
+    from tests.test_gpu_parity import _packed
+
+    game = map_name_to_scenario(name, conflict_strategy=ConflictStrategy.CANCEL_BOTH, max_cycles=400)
+    o, b = Oracle(game), game.bucket
+    free = int((~game.terrain.reshape(-1)).sum())
+    most = min(free * 3 // 4, 2 * b.per_player_capacity - 20)
+    extra = [most * k // 11 for k in range(12)]
+    st = _packed(game, extra, seed=6)
+    assert (o.violations(st) == 0).all()
+    L, C = len(extra), b.per_player_capacity
+    for bot in (WORKER_RUSH, BARRACKS_RUSH):
+        print(f"crowded searches {name} {bot}", flush=True)
+        seat = _seat_env(game, False, bot)
+        ref, carry = copy_state(st), empty_carry(L, C)
+        for t in range(24):
+            if t % 8 == 0:
+                for player in (0, 1):
+                    want_carry = copy_state(carry)
+                    want = o.abstraction_act(copy_state(ref), want_carry, bot, LIGHT, player)
+                    dev_carry = _carry_to_device(carry, seat.device)
+                    got = bots.abstraction_act(seat.env, to_device(seat.env, ref), dev_carry,
+                                               bots.Bot("probe", bot, LIGHT), player)
+                    for field, w in want.items():
+                        np.testing.assert_array_equal(got[field].cpu().numpy(), w, err_msg=f"{name} {t} {player} {field}")
+                    _assert_carry_equal(want_carry, _carry_to_host(dev_carry), f"{name} {t} {player}")
+            o.seat_step(ref, carry, bot, LIGHT, 0, _learner_actions(o, ref, t), False, observe=False)
+        sst = SeatState(to_device(seat.env, st), _carry_to_device(empty_carry(L, C), seat.device),
+                        torch.zeros(L, dtype=torch.int32, device=seat.device))
+        seat.rollout(sst, 24, (41, 43), record=False)
+        assert_states_equal(ref, to_host(sst.environment_state), f"{name} fused")
+        _assert_carry_equal(carry, _carry_to_host(sst.carry), f"{name} fused")
