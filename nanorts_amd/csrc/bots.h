@@ -8,8 +8,9 @@
 // (after the env block) holds the carry (AbstractActions rows), the plan of
 // each unit, candidate lists and the search scratch.  Decisions are per unit,
 // one lane per own slot; the walk over the queued units is sequential as in
-// the reference (each search sees the cells claimed before it), and each
-// search runs on lane 0 over LDS stacks.
+// the reference (each search sees the cells claimed before it); the searches'
+// straight paths run a lane each, the others one by one over LDS stacks, on
+// the lane of their unit (a lane per direction measured the same: 11.9 ms).
 #pragma once
 
 #include "engine.h"
@@ -542,7 +543,7 @@ NR_DEV void barracks_rush(const KGame& g, const Hdr& h, const Env& e, Bot& b, co
 }
 
 // ---------------------------------------------------------------------------
-// pathfinding.search (N/bots/pathfinding.py:170-245) on lane 0.
+// pathfinding.search (N/bots/pathfinding.py:170-245) on one lane.
 // Open cells pop by least f = g + Manhattan(cell, target), the most recently
 // inserted first among equal f; neighbours are inserted up, right, down,
 // left; each cell once.  A neighbour's f is the popped cell's f or f + 2,
@@ -951,9 +952,9 @@ NR_DEV bool reaches(const KGame& g, const AS3 uint32_t* open, int32_t start, int
 // 904-952): returns how many desires it keeps.  Each queued unit has a lane,
 // and the searches' straight paths run side by side; a unit that claims a cell
 // closes it for the searches after it, and those whose path held that cell
-// walk again before the next answer that needs it.  A search with a dead end
-// alone takes the stacks, and only where the flood says that its goal can be
-// reached at all.  50 fused cycles of 32768 games against WorkerRush on 16x16
+// walk again before the next answer that needs it.  Only a search that meets a
+// dead end takes the stacks, and only where the flood says that its goal can
+// be reached at all.  50 fused cycles of 32768 games against WorkerRush on 16x16
 // took 16.5 ms with every search whole on lane 0 (a search for an enclosed
 // goal there popped the whole board, about 50 k cycles of a wave), 11.7 ms so.
 template <int TW = kWave>

@@ -1074,6 +1074,7 @@ NR_DEV int32_t order_requests(const KGame& g, const Env& e, int lane, int32_t* n
     for (int32_t i = lane; i < n; i += kWave) {
         const uint64_t ki = keys[i];
         int32_t pos = 0;
+#pragma unroll 4
         for (int32_t j = 0; j < n; ++j) {
             const uint64_t kj = keys[j];
             pos += (kj < ki) || (kj == ki && j < i);
@@ -1135,6 +1136,7 @@ NR_DEV int32_t order_requests(const KGame& g, const Env& e, int lane, int32_t* n
     for (int32_t i = lane; i < no; i += kWave) {
         const uint64_t ki = keys[i];
         int32_t pos = 0;
+#pragma unroll 4
         for (int32_t j = 0; j < no; ++j) pos += keys[j] < ki;
         rank[nr + pos] = (int16_t)(N + tmp[i]);
     }

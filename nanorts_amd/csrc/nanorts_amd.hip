@@ -695,20 +695,43 @@ bool state_complete(const nanorts_state& s) {
     if (l >= lanes) return;                                                       \
     const Env e = env_view(g, lds + g.lay.hdr_bytes + wave * g.lay.env_bytes);
 
-// Canonical commands from the reference's int32 Commands operands.
+// Canonical commands from the reference's int32 Commands operands, for the
+// live units (no other position's command is read): the loads of kSets
+// positions a lane are issued before the first is used, and positions without
+// a unit all read the row's first word, so that only lines with a unit's
+// command are fetched.  4 x 16384 games on 16x16 (140 positions): 417 us with
+// every position loaded, 64 at a time, 398 us so.
 NR_DEV void stage_commands(const KGame& g, const Env& e, int64_t l, const nanorts_commands& c, int lane) {
+    constexpr int kSets = 3;
     const Layout& y = g.lay;
     const int32_t owned = 2 * g.C;
     const int32_t top = (1 << g.rank_bits) - 1;
-    for (int32_t p = lane; p < owned; p += kWave) {
-        const int64_t i = l * owned + p;
-        at<int8_t>(e, y.c_kind)[p] = (int8_t)canon_kind(c.kind[i]);
-        at<int8_t>(e, y.c_dir)[p] = (int8_t)canon_dir(c.direction[i]);
-        at<int8_t>(e, y.c_ptype)[p] = (int8_t)canon_ptype(c.produced_type[i], g.T);
-        at<int16_t>(e, y.c_target)[p] = (int16_t)canon_target(c.target_cell[i], g.cells);
-        at<int32_t>(e, y.c_none)[p] = c.none_duration[i];
-        const int32_t ro = c.request_order[i];
-        at<int16_t>(e, y.c_rank)[p] = (int16_t)clampi(ro == kAbsent ? 0 : ro, 0, top);
+    for (int32_t base = 0; base < owned; base += kSets * kWave) {
+        bool live[kSets];
+        int32_t kind[kSets], dir[kSets], ptype[kSets], target[kSets], none[kSets], ro[kSets];
+#pragma unroll
+        for (int k = 0; k < kSets; ++k) {
+            const int32_t p = base + k * kWave + lane;
+            live[k] = p < owned && e.birth[g.N + (p < owned ? p : 0)] != kAbsent;
+            const int64_t i = l * owned + (live[k] ? p : 0);
+            kind[k] = c.kind[i];
+            dir[k] = c.direction[i];
+            ptype[k] = c.produced_type[i];
+            target[k] = c.target_cell[i];
+            none[k] = c.none_duration[i];
+            ro[k] = c.request_order[i];
+        }
+#pragma unroll
+        for (int k = 0; k < kSets; ++k) {
+            const int32_t p = base + k * kWave + lane;
+            if (!live[k]) continue;
+            at<int8_t>(e, y.c_kind)[p] = (int8_t)canon_kind(kind[k]);
+            at<int8_t>(e, y.c_dir)[p] = (int8_t)canon_dir(dir[k]);
+            at<int8_t>(e, y.c_ptype)[p] = (int8_t)canon_ptype(ptype[k], g.T);
+            at<int16_t>(e, y.c_target)[p] = (int16_t)canon_target(target[k], g.cells);
+            at<int32_t>(e, y.c_none)[p] = none[k];
+            at<int16_t>(e, y.c_rank)[p] = (int16_t)clampi(ro[k] == kAbsent ? 0 : ro[k], 0, top);
+        }
     }
     wave_sync();
 }
