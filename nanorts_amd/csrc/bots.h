@@ -38,7 +38,7 @@ struct BotLayout {
     // carry rows [C]
     int32_t k_kind, k_ubirth, k_order, k_target, k_tbirth, k_base, k_bbirth, k_cell, k_utype, k_trained;
     // per unit [C]
-    int32_t u_flags, u_role, u_rank, u_es, u_eb, u_goal, u_radius;
+    int32_t u_flags, u_role, u_rank, u_es, u_goal, u_radius;
     int32_t u_fkind, u_fdir, u_ftarget, u_fptype, u_fclaimed, u_fcost;
     int32_t u_sel, u_dir, u_drank, u_queue;
     int32_t u_live, u_lbirth, u_list, u_lkey;  // live units and their births; a scratch list with keys
@@ -64,7 +64,13 @@ struct Bot {
     AS3 uint8_t* base;
     int32_t player, block;
     int32_t n_enemy, n_resource, n_stock;
-    int32_t n_live;  // own units present, listed in u_live
+    int32_t n_live;  // own units present, listed in u_live by birth
+    // the lane's first live unit (u_live[lane]), from bot_begin through the
+    // rush decisions: its birth, its cell with its nearest enemy's slot above
+    // bit 16, and its slot in the block (bits 0..9), type (10..13), whether it
+    // is available (14) and carries (15) and its role bits (from 16): three
+    // registers, because the half-wave kernel has few left
+    int32_t own_birth, own_places, own_bits;
     int32_t next_order;
     int32_t reserved0, reserved1;  // pending production cost per player
 };
@@ -124,6 +130,14 @@ NR_DEV int32_t team_sum(int32_t v) {
     return v;
 }
 
+// The same where few lanes hold other than 0.
+template <int TW = kWave>
+NR_DEV int32_t team_sum_few(int32_t v) {
+    int32_t sum = 0;
+    for (uint64_t m = tballot<TW>(v != 0); m != 0ull; m &= m - 1ull) sum = wadd(sum, tread<TW>(v, (int32_t)__builtin_ctzll(m)));
+    return sum;
+}
+
 NR_DEV int32_t bit_of(const AS3 uint32_t* m, int32_t c) { return (int32_t)((m[c >> 5] >> (c & 31)) & 1u); }
 NR_DEV void set_bit(AS3 uint32_t* m, int32_t c) { __atomic_fetch_or(&m[c >> 5], 1u << (c & 31), __ATOMIC_RELAXED); }
 
@@ -149,6 +163,38 @@ NR_DEV Unit unit_at(const KGame& g, const Env& e, const Bot& b, int32_t i) {
     u.present = u.birth != kAbsent;
     u.available = u.present && e.pkind[u.slot] == kAbsent;
     return u;
+}
+
+// The k-th live unit (k = lane, lane + TW, ...), its block slot in *i: the
+// first of a lane comes from registers, which took most of the LDS round trips
+// out of the rush decisions (each read live list, unit and role again).  Of
+// what it carries a lane's first only knows whether it carries.
+NR_DEV Unit live_unit(const KGame& g, const Env& e, const Bot& b, const BotLayout& y, int32_t k, int lane, int32_t* i) {
+    if (k != lane) {
+        *i = bv<int16_t>(b, y.u_live)[k];
+        return unit_at(g, e, b, *i);
+    }
+    *i = b.own_bits & 1023;
+    Unit u;
+    u.slot = b.block + *i;
+    u.birth = b.own_birth;
+    u.cell = (int16_t)b.own_places;
+    u.type = (b.own_bits >> 10) & 15;
+    u.carried = (b.own_bits >> 15) & 1;
+    u.present = true;
+    u.available = ((b.own_bits >> 14) & 1) != 0;
+    return u;
+}
+NR_DEV int32_t live_slot(const Bot& b, const BotLayout& y, int32_t k, int lane) {
+    return k == lane ? b.own_bits & 1023 : (int32_t)bv<int16_t>(b, y.u_live)[k];
+}
+// Its role bits (u_role past a lane's first).
+NR_DEV int32_t live_role(const Bot& b, const BotLayout& y, int32_t k, int32_t i, int lane) {
+    return k == lane ? b.own_bits >> 16 : (int32_t)bv<uint8_t>(b, y.u_role)[i];
+}
+NR_DEV void set_live_role(Bot& b, const BotLayout& y, int32_t k, int32_t i, int lane, int32_t role) {
+    if (k == lane) b.own_bits = (b.own_bits & 0xFFFF) | (role << 16);
+    else bv<uint8_t>(b, y.u_role)[i] = (uint8_t)role;
 }
 
 // Manhattan-nearest slot of a candidate list, ties by the lowest birth then
@@ -209,6 +255,8 @@ NR_DEV void bot_begin(const KGame& g, const Hdr& h, const Env& e, Bot& b, const 
     // live own units in slot order, with their births
     AS3 int16_t* live = bv<int16_t>(b, y.u_live);
     AS3 int32_t* lbirth = bv<int32_t>(b, y.u_lbirth);
+    AS3 int16_t* found = bv<int16_t>(b, y.u_list);
+    AS3 int32_t* fbirth = bv<int32_t>(b, y.u_lkey);
     int32_t n = 0;
     for (int32_t i0 = 0; i0 < C; i0 += TW) {
         const int32_t i = i0 + lane;
@@ -216,8 +264,8 @@ NR_DEV void bot_begin(const KGame& g, const Hdr& h, const Env& e, Bot& b, const 
         const bool present = bi != kAbsent;
         const uint64_t m = tballot<TW>(present);
         if (present) {
-            live[n + tcount_below<TW>(m)] = (int16_t)i;
-            lbirth[n + tcount_below<TW>(m)] = bi;
+            found[n + tcount_below<TW>(m)] = (int16_t)i;
+            fbirth[n + tcount_below<TW>(m)] = bi;
         }
         n += popc(m);
     }
@@ -266,18 +314,37 @@ NR_DEV void bot_begin(const KGame& g, const Hdr& h, const Env& e, Bot& b, const 
     b.n_resource = nr_ < g.N ? nr_ : g.N;
     b.n_stock = ns < C ? ns : C;
     wave_sync();
-    // birth rank among the present units (abstraction._rank) and the
-    // nearest enemy of every live unit
+    // birth rank among the present units (abstraction._rank), which orders the
+    // live list (equal births, which no valid state has, by slot)
     for (int32_t k = lane; k < n; k += TW) {
-        const int32_t i = live[k], bi = lbirth[k];
-        int32_t r = 0;
+        const int32_t i = found[k], bi = fbirth[k];
+        int32_t r = 0, at = 0;
 #pragma unroll 4
-        for (int32_t q = 0; q < n; ++q) r += lbirth[q] < bi ? 1 : 0;
+        for (int32_t q = 0; q < n; ++q) {
+            const int32_t bq = fbirth[q];
+            r += bq < bi ? 1 : 0;
+            at += (bq < bi || (bq == bi && q < k)) ? 1 : 0;
+        }
         bv<int16_t>(b, y.u_rank)[i] = (int16_t)r;
+        live[at] = (int16_t)i;
+        lbirth[at] = bi;
+    }
+    wave_sync();
+    // the nearest enemy of every live unit
+    b.own_birth = kAbsent;
+    b.own_places = b.own_bits = 0;
+    for (int32_t k = lane; k < n; k += TW) {
+        const int32_t i = live[k];
+        const Unit u = unit_at(g, e, b, i);
         int32_t es, eb;
-        closest(g, e, e.cell[b.block + i], le, ne, &es, &eb);
-        bv<int16_t>(b, y.u_es)[i] = (int16_t)es;
-        bv<int32_t>(b, y.u_eb)[i] = eb;
+        closest(g, e, u.cell, le, ne, &es, &eb);
+        if (k == lane) {
+            b.own_birth = u.birth;
+            b.own_places = (u.cell & 0xFFFF) | (es << 16);
+            b.own_bits = i | (u.type << 10) | (u.available ? 1 << 14 : 0) | (u.carried > 0 ? 1 << 15 : 0);
+        } else {
+            bv<int16_t>(b, y.u_es)[i] = (int16_t)es;
+        }
     }
     wave_sync();
 }
@@ -316,28 +383,23 @@ NR_DEV int32_t building_site(const KGame& g, const Hdr& h, const Env& e, const B
 // Per-unit role bits of the rush decisions (u_role, one byte per own slot).
 enum : uint8_t { R_WORKER = 1, R_PICK = 2, R_IDLE = 4, R_LAST = 8 };
 
-NR_DEV AS3 uint8_t* roles(const Bot& b, const BotLayout& y) { return bv<uint8_t>(b, y.u_role); }
-
 // The unit of least birth among those whose role byte has any of `bits`
 // (rush.first_in_unit_order, N/bots/rush.py:56-58), excluding `skip0` and
 // `skip1`; -1 when there is none.
 template <int TW = kWave>
 NR_DEV int32_t first_of(const KGame& g, const Env& e, const Bot& b, const BotLayout& y, uint8_t bits, int32_t skip0,
                         int32_t skip1, int lane) {
-    const AS3 uint8_t* r = roles(b, y);
-    int32_t best = kLast, who = -1;
-    for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        if (!(r[i] & bits) || i == skip0 || i == skip1) continue;
-        const int32_t bi = e.birth[b.block + i];
-        if (bi < best) {
-            best = bi;
-            who = i;
-        }
+    // the live list is ordered by birth: the first match is the least
+    const int32_t most = tmax<TW>(b.n_live);
+    int32_t first = -1;
+    for (int32_t base = 0; base < most; base += TW) {
+        const int32_t k = base + lane;
+        const int32_t i = k < b.n_live ? live_slot(b, y, k, lane) : -1;
+        const bool match = i >= 0 && (live_role(b, y, k, i, lane) & bits) && i != skip0 && i != skip1;
+        const uint64_t m = tballot<TW>(match);
+        if (first < 0 && m != 0ull) first = tread<TW>(i, (int32_t)__builtin_ctzll(m));
     }
-    const int32_t mn = team_min<TW>(best);
-    const uint64_t at = tballot<TW>(who >= 0 && best == mn);
-    return at == 0ull ? -1 : tread<TW>(who, (int32_t)__builtin_ctzll(at));
+    return first;
 }
 
 // abstraction.build_if_not_already_building (N/bots/abstraction.py:286-297)
@@ -371,8 +433,8 @@ NR_DEV int32_t build_base(const KGame& g, const Hdr& h, const Env& e, Bot& b, co
     for (int32_t w = lane; w < (g.cells + 31) / 32; w += TW) reserved[w] = 0u;
     bool any_base = false;
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const Unit u = unit_at(g, e, b, i);
+        int32_t i;
+        const Unit u = live_unit(g, e, b, y, k, lane, &i);
         any_base |= u.present && u.type == kTypeBase;
     }
     any_base = tballot<TW>(any_base) != 0ull;
@@ -388,14 +450,13 @@ NR_DEV int32_t build_base(const KGame& g, const Hdr& h, const Env& e, Bot& b, co
 // idle ones (no site to harvest) R_IDLE.
 template <int TW = kWave>
 NR_DEV void harvest(const KGame& g, const Env& e, Bot& b, const BotLayout& y, int lane) {
-    AS3 uint8_t* r = roles(b, y);
     const AS3 int16_t* lr = bv<int16_t>(b, y.l_resource);
     const AS3 int16_t* ls = bv<int16_t>(b, y.l_stock);
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const uint8_t role = r[i];
+        int32_t i;
+        const Unit u = live_unit(g, e, b, y, k, lane, &i);
+        const int32_t role = live_role(b, y, k, i, lane);
         if (!(role & R_PICK)) continue;
-        const Unit u = unit_at(g, e, b, i);
         int32_t rs, rb, ss, sb;
         closest(g, e, u.cell, lr, b.n_resource, &rs, &rb);
         closest(g, e, u.cell, ls, b.n_stock, &ss, &sb);
@@ -408,7 +469,7 @@ NR_DEV void harvest(const KGame& g, const Env& e, Bot& b, const BotLayout& y, in
         if (occupied && !unchanged)
             put_unit<TW>(g, b, u, i, false, kAbHarvest, carrying ? kAbsent : rs, carrying ? kAbsent : rb, ss, sb, kAbsent,
                      kAbsent, y);
-        if (!occupied) r[i] = (uint8_t)(role | R_IDLE);
+        if (!occupied) set_live_role(b, y, k, i, lane, role | R_IDLE);
     }
     b.next_order = wadd(b.next_order, g.C + 1);
     wave_sync();
@@ -418,16 +479,14 @@ NR_DEV void harvest(const KGame& g, const Env& e, Bot& b, const BotLayout& y, in
 // any of `bits`; R_LAST units are stamped last.
 template <int TW = kWave>
 NR_DEV void attack_nearest(const KGame& g, const Env& e, Bot& b, const BotLayout& y, uint8_t bits, int lane) {
-    const AS3 uint8_t* r = roles(b, y);
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const uint8_t role = r[i];
+        int32_t i;
+        const Unit u = live_unit(g, e, b, y, k, lane, &i);
+        const int32_t role = live_role(b, y, k, i, lane);
         if (!(role & bits)) continue;
-        const int32_t es = bv<int16_t>(b, y.u_es)[i];
+        const int32_t es = k == lane ? b.own_places >> 16 : (int32_t)bv<int16_t>(b, y.u_es)[i];
         if (es == kAbsent) continue;
-        const Unit u = unit_at(g, e, b, i);
-        put_unit<TW>(g, b, u, i, (role & R_LAST) != 0, kAbAttack, es, bv<int32_t>(b, y.u_eb)[i], kAbsent, kAbsent,
-                 kAbsent, kAbsent, y);
+        put_unit<TW>(g, b, u, i, (role & R_LAST) != 0, kAbAttack, es, e.birth[es], kAbsent, kAbsent, kAbsent, kAbsent, y);
     }
     b.next_order = wadd(b.next_order, g.C + 1);
     wave_sync();
@@ -438,8 +497,8 @@ template <int TW, typename Pick>
 NR_DEV void train_where(const KGame& g, const Env& e, Bot& b, const BotLayout& y, int32_t unit_type, Pick pick,
                         int lane) {
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const Unit u = unit_at(g, e, b, i);
+        int32_t i;
+        const Unit u = live_unit(g, e, b, y, k, lane, &i);
         if (pick(u)) put_unit<TW>(g, b, u, i, false, kAbTrain, kAbsent, kAbsent, kAbsent, kAbsent, kAbsent, unit_type, y);
     }
     b.next_order = wadd(b.next_order, g.C + 1);
@@ -450,13 +509,12 @@ NR_DEV void train_where(const KGame& g, const Env& e, Bot& b, const BotLayout& y
 // marks the workers (present units that can harvest) R_WORKER.
 template <int TW = kWave>
 NR_DEV void melee_attack(const KGame& g, const Hdr& h, const Env& e, Bot& b, const BotLayout& y, int lane) {
-    AS3 uint8_t* r = roles(b, y);
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const Unit u = unit_at(g, e, b, i);
+        int32_t i;
+        const Unit u = live_unit(g, e, b, y, k, lane, &i);
         const bool harvests = type_flag(g, h, u.type, FL_HARVEST);
         const bool melee = u.present && type_flag(g, h, u.type, FL_ATTACK) && !harvests && u.available;
-        r[i] = (uint8_t)((melee ? R_PICK : 0) | ((u.present && harvests) ? R_WORKER : 0));
+        set_live_role(b, y, k, i, lane, (melee ? R_PICK : 0) | ((u.present && harvests) ? R_WORKER : 0));
     }
     wave_sync();
     attack_nearest<TW>(g, e, b, y, R_PICK, lane);
@@ -465,14 +523,13 @@ NR_DEV void melee_attack(const KGame& g, const Hdr& h, const Env& e, Bot& b, con
 // Role bytes for a new decision: R_WORKER kept, `pick` units get R_PICK,
 // others lose R_PICK / R_IDLE / R_LAST.
 template <int TW = kWave>
-NR_DEV void mark_picks(const KGame& g, const Bot& b, const BotLayout& y, int32_t skip0, int32_t skip1, int32_t only,
+NR_DEV void mark_picks(const KGame& g, Bot& b, const BotLayout& y, int32_t skip0, int32_t skip1, int32_t only,
                        int lane) {
-    AS3 uint8_t* r = roles(b, y);
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const uint8_t w = r[i] & R_WORKER;
+        const int32_t i = live_slot(b, y, k, lane);
+        const int32_t w = live_role(b, y, k, i, lane) & R_WORKER;
         const bool pick = only >= 0 ? i == only : (w && i != skip0 && i != skip1);
-        r[i] = (uint8_t)(w | (pick ? R_PICK : 0));
+        set_live_role(b, y, k, i, lane, w | (pick ? R_PICK : 0));
     }
     wave_sync();
 }
@@ -492,13 +549,12 @@ NR_DEV void worker_rush(const KGame& g, const Hdr& h, const Env& e, Bot& b, cons
     harvest<TW>(g, e, b, y, lane);
     // free = (workers - builder - harvester) | idle harvester; the idle
     // harvester is stamped last
-    AS3 uint8_t* r = roles(b, y);
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const uint8_t role = r[i];
+        const int32_t i = live_slot(b, y, k, lane);
+        const int32_t role = live_role(b, y, k, i, lane);
         const bool idle = (role & R_IDLE) != 0;
         const bool free = ((role & R_WORKER) && i != builder && i != harvester) || idle;
-        r[i] = (uint8_t)((role & R_WORKER) | (free ? R_PICK : 0) | (idle ? R_LAST : 0));
+        set_live_role(b, y, k, i, lane, (role & R_WORKER) | (free ? R_PICK : 0) | (idle ? R_LAST : 0));
     }
     wave_sync();
     attack_nearest<TW>(g, e, b, y, R_PICK, lane);
@@ -514,8 +570,8 @@ NR_DEV void barracks_rush(const KGame& g, const Hdr& h, const Env& e, Bot& b, co
     int32_t held = 0;
     bool any_barracks = false;
     for (int32_t k = lane; k < b.n_live; k += TW) {
-        const int32_t i = bv<int16_t>(b, y.u_live)[k];
-        const Unit u = unit_at(g, e, b, i);
+        int32_t i;
+        const Unit u = live_unit(g, e, b, y, k, lane, &i);
         held += (u.present && u.type == kTypeWorker) ? 1 : 0;
         any_barracks |= u.present && u.type == kTypeBarracks;
     }
@@ -760,7 +816,6 @@ NR_DEV int32_t translate_plan(const KGame& g, const Hdr& h, const Env& e, Bot& b
     AS3 uint32_t* freem = bv<uint32_t>(b, y.m_free);
     for (int32_t w = lane; w < words; w += TW) {
         claimed[w] = 0u;
-        freem[w] = 0u;
     }
     wave_sync();
     // _pending_usage (N/bots/abstraction.py:331-359)
@@ -779,12 +834,22 @@ NR_DEV int32_t translate_plan(const KGame& g, const Hdr& h, const Env& e, Bot& b
             else cost1 = wadd(cost1, c);
         }
     }
-    b.reserved0 = team_sum<TW>(cost0);
-    b.reserved1 = team_sum<TW>(cost1);
+    b.reserved0 = team_sum_few<TW>(cost0);
+    b.reserved1 = team_sum_few<TW>(cost1);
     wave_sync();
     // _free_cells (:362-365)
-    for (int32_t c = lane; c < g.cells; c += TW)
-        if (h.terrain[c] == 0 && e.entity[c] == kAbsent && !bit_of(claimed, c)) set_bit(freem, c);
+    // a ballot a word: TW cells at a time (a bit set by LDS atomics for each cell
+    // waited on memory for every round of them)
+    const int32_t rounds = (g.cells + TW - 1) / TW;
+#pragma unroll 2
+    for (int32_t k = 0; k < rounds; ++k) {
+        const int32_t c = k * TW + lane;
+        const bool on = c < g.cells;
+        const bool open = on && h.terrain[on ? c : 0] == 0 && e.entity[on ? c : 0] == kAbsent;
+        const uint64_t m = tballot<TW>(open);
+        const int32_t w = k * (TW / 32) + lane;
+        if (lane < TW / 32 && w < words) freem[w] = (uint32_t)(m >> (32 * lane)) & ~claimed[w];
+    }
     wave_sync();
     // _standing (:383-423) and _plan (:653-715) with _fallback (:575-650)
     for (int32_t i = lane; i < C; i += TW) {

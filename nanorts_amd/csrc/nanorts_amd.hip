@@ -595,7 +595,6 @@ bool shape_for_bots(const nanorts_game* game, Shape* out, BotLayout* by, std::st
     const int32_t scratch = o;
     by->u_rank = take(2 * C);
     by->u_es = take(2 * C);
-    by->u_eb = take(4 * C);
     by->u_role = take(C);
     by->u_list = take(2 * C);
     by->l_enemy = take(2 * C);
