@@ -430,7 +430,8 @@ int nanorts_amd_env_transition(void* stream, const nanorts_game* game, nanorts_s
  * `taken` (int32[L] work words of the caller, or NULL) lets a call of many
  * games run as two launches: a first pass with two games per wave, which
  * leaves in taken[l] whether it stepped game l, and a second for the rest;
- * the results are the same. */
+ * the results are the same.  The environment variable NANORTS_AMD_FIRST_PASS
+ * set to "pair" takes the two launches however few the games, "lean" the one. */
 int nanorts_amd_env_step_from(void* stream, const nanorts_game* game, nanorts_state from, nanorts_state state,
                               int64_t lanes, const int32_t* actions0, const int32_t* actions1, int64_t action_stride,
                               int32_t partial, int32_t reset, nanorts_env_results results, int32_t* taken);

@@ -477,6 +477,18 @@ bool few_games(int64_t lanes, int32_t cells) {
     return lanes <= (int64_t)(cells >= 4 * kWave ? 16 : 8) * cus;
 }
 
+// The first pass that the environment variable NANORTS_AMD_FIRST_PASS asks
+// for, whatever the board and the games: "lean" one game per wave (env.step and
+// the seat rollout have no such pass and run one launch), "pair" two.
+enum class ForcedPass { kNone, kLean, kPair };
+ForcedPass forced_first_pass() {
+    const char* mode = std::getenv("NANORTS_AMD_FIRST_PASS");
+    if (!mode) return ForcedPass::kNone;
+    return std::strcmp(mode, "lean") == 0   ? ForcedPass::kLean
+           : std::strcmp(mode, "pair") == 0 ? ForcedPass::kPair
+                                            : ForcedPass::kNone;
+}
+
 // A smaller env block for the kernels that read a few leaves: `masks` holds
 // the leaves the legality rows read, the occupancy bitmaps and the staged
 // words (k_legality); otherwise the block is empty (the samplers read only
@@ -3653,12 +3665,15 @@ static int env_step(void* stream, const nanorts_game* game, const nanorts_state&
         return fail(NANORTS_INVALID_ARGUMENT, std::string(call) + " needs environment_root and episode_index");
     if (reset && !state_complete(game->initial)) return fail(NANORTS_INVALID_ARGUMENT, "game->initial is incomplete");
     // Two passes where the caller gives the work words and the games are many
-    // (see k_env_step_pair); the second steps what the first left.
+    // (see k_env_step_pair), or NANORTS_AMD_FIRST_PASS=pair asks for them; the
+    // second steps what the first left.
     Shape pair;
     std::string why;
-    const bool paired = taken && lanes > 0 && !few_games(lanes, game->cells) &&
+    const ForcedPass forced = forced_first_pass();
+    const bool paired = taken && lanes > 0 && forced != ForcedPass::kLean &&
+                        (forced == ForcedPass::kPair || !few_games(lanes, game->cells)) &&
                         ((((uintptr_t)results.feature_maps) | ((uintptr_t)results.final_feature_maps)) & 7u) == 0 &&
-                        shape_for_first_pass(game, true, false, &pair, &why);
+                        shape_for_first_pass(game, true, forced == ForcedPass::kPair, &pair, &why);
     if (paired) {
         EnvStepArgs args;
         std::memset(&args, 0, sizeof(args));
@@ -4047,10 +4062,9 @@ static int choose_first_pass(const nanorts_game* game, const Shape& full, int64_
     if (!full.g.fast_obs || !shape_for_first_pass(game, false, false, lean, &why) ||
         games_per_cu(lean->g.lay, lean->wpb, kLeanWavesPerSimd) < games_per_cu(full.g.lay, full.wpb, 4))
         return 0;
-    const char* mode = std::getenv("NANORTS_AMD_FIRST_PASS");
-    const bool want_lean = mode && std::strcmp(mode, "lean") == 0;
-    const bool want_pair = mode && std::strcmp(mode, "pair") == 0;
-    if (want_lean || (!want_pair && lanes > 0 && few_games(lanes, game->cells))) return 1;
+    const ForcedPass forced = forced_first_pass();
+    const bool want_pair = forced == ForcedPass::kPair;
+    if (forced == ForcedPass::kLean || (!want_pair && lanes > 0 && few_games(lanes, game->cells))) return 1;
     return shape_for_first_pass(game, true, want_pair, pair, &why) ? 2 : 1;
 }
 
@@ -4337,9 +4351,8 @@ static int seat_rollout(void* stream, const nanorts_game* game, nanorts_state st
     // keeps the one pass
     Shape ps;
     BotArgs pa;
-    const char* mode = std::getenv("NANORTS_AMD_FIRST_PASS");
     const bool paired = results.progress != nullptr && (((uintptr_t)results.feature_maps) & 7u) == 0 &&
-                        !(mode && std::strcmp(mode, "lean") == 0) &&
+                        forced_first_pass() != ForcedPass::kLean &&
                         seat_pair_shape(game, strategy, trained_type, carry, sh, &ps, &pa);
     const int64_t pair_blocks = paired ? (lanes + 2 * ps.wpb - 1) / (2 * ps.wpb) : 0;
     for (int32_t t0 = 0; t0 < steps; t0 += kRolloutChunk) {

@@ -143,6 +143,7 @@ def test_env_step_of_many_games_in_two_passes(name, L, partial, monkeypatch):
     from nanorts_amd import env as envmod
     from tests.helpers import to_device
     from tests.test_gpu_parity import _packed
+    from tests.test_gpu_step_two_passes import two_pass_step
 
     _say(f"two-pass env.step {name}")
     game = map_name_to_scenario(name, max_cycles=44, conflict_strategy="CANCEL_RANDOM")
@@ -155,9 +156,11 @@ def test_env_step_of_many_games_in_two_passes(name, L, partial, monkeypatch):
         state.core_state.leaves[k][:7] = v
         state.core_state.leaves[k][-3:] = v[-3:]
     env.rollout(state, 36, (5, 6), record=False)
-    ends = 0
+    seen, ends = set(), 0
     for t in range(12):
         actions = env.sample_actions(env.get_avail_actions(state, form="words"), (7, 8), t)
+        *_, taken = two_pass_step(env, state, actions)
+        seen |= set(taken.tolist())
         with monkeypatch.context() as m:
             m.setattr(envmod, "_FEW_GAMES", 1 << 40)
             want = env.step(None, state.clone(), actions, donate=True)
@@ -167,7 +170,7 @@ def test_env_step_of_many_games_in_two_passes(name, L, partial, monkeypatch):
         _same(before, state)
         _same(want, env.step(None, state, actions, donate=True))
         ends += int(want[3]["__all__"].sum())
-    assert ends > 0
+    assert seen == {0, 1} and ends > 0  # both launches stepped games
 
 
 @pytest.mark.parametrize("name,L", BOARDS[:3])
