@@ -894,16 +894,18 @@ NR_DEV void store_window_rows(const KGame& g, const nanorts_state& s, int64_t l,
     store_scalars(s, l, e, lane);
 }
 
-// The slots outside the window, row l of `from` into row l of `s`: a first
-// pass that writes another state than it read has only the window staged.
+// The slots outside the window, row `l_from` of `from` into row l of `s`: a
+// first pass that writes another state than it read, or resets a game, has
+// only the window staged.
 template <int TW>
-NR_DEV void copy_gap_rows(const KGame& g, const nanorts_state& from, const nanorts_state& s, int64_t l, int lane) {
+NR_DEV void copy_gap_rows(const KGame& g, const nanorts_state& from, int64_t l_from, const nanorts_state& s, int64_t l,
+                          int lane) {
     const int32_t N = g.N, C = g.C, E = g.E, sh = g.shift;
-    const int64_t row = l * (int64_t)(E + 2 * sh);
+    const int64_t all = E + 2 * sh;
     for (int32_t i = lane; i < 2 * sh; i += TW) {
-        const int64_t at = row + (i < sh ? N + C + i : E + i);
-#define NR_GAP(flag, field, member, type, count) const type v_##member = from.field[at];
-#define NR_GAP_OUT(flag, field, member, type, count) s.field[at] = v_##member;
+        const int64_t slot = i < sh ? N + C + i : E + i;
+#define NR_GAP(flag, field, member, type, count) const type v_##member = from.field[l_from * all + slot];
+#define NR_GAP_OUT(flag, field, member, type, count) s.field[l * all + slot] = v_##member;
         NR_SLOT_LEAVES(NR_GAP)
         NR_SLOT_LEAVES(NR_GAP_OUT)
 #undef NR_GAP

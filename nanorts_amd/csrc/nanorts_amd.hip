@@ -2138,6 +2138,7 @@ __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_env_step_pair(EnvS
     no_request(q);
     int lane, team;
     int64_t l;
+    bool restarts = false;
     {
         const EnvStepArgs& a = fresh_env_step_args();
         const KGame& g = a.g;
@@ -2207,7 +2208,8 @@ __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_env_step_pair(EnvS
         const Outcome oc = decide_counted<TW>(e, lane);
         // a game that ends takes the initial state, which has to fit the window
         // too; nothing has been written yet
-        if (a.reset != 0 && g.shift > 0 && (oc.over != 0 || time >= g.max_cycles) && !initial_fits_window<TW>(g, lane)) {
+        restarts = a.reset != 0 && (oc.over != 0 || time >= g.max_cycles);
+        if (restarts && g.shift > 0 && !initial_fits_window<TW>(g, lane)) {
             if (lane == 0) a.taken[l] = 0;
             return;
         }
@@ -2225,7 +2227,10 @@ __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_env_step_pair(EnvS
         const Env e = team_env(g, team);
         if (g.shift > 0) {
             store_window_rows<TW>(g, a.s, l, e, lane);
-            if (a.elsewhere != 0) copy_gap_rows<TW>(g, a.from, a.s, l, lane);
+            // (an empty slot's other leaves are part of the state too: a game
+            // that restarts takes the initial state's)
+            if (restarts) copy_gap_rows<TW>(g, g.initial, 0, a.s, l, lane);
+            else if (a.elsewhere != 0) copy_gap_rows<TW>(g, a.from, l, a.s, l, lane);
         } else {
             store_env<TW>(g, a.s, l, e, lane);
         }

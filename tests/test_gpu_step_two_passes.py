@@ -125,3 +125,37 @@ def test_two_passes_match_one(name, surface, monkeypatch):
         ends += int(want[3]["__all__"].sum())
         state = want[1]
     assert seen == {0, 1} and ends > 0
+
+
+@pytest.mark.parametrize("donate", [True, False])
+def test_restart_replaces_every_slot(donate, monkeypatch):
+    """A game that ends takes the whole initial state: also slots outside the
+    first pass's window, whose leaves a program may have left other than the
+    initial state has them (here five leaves of empty slots); a game that goes
+    on keeps them."""
+    import nanorts_amd
+    from nanorts_amd import env as envmod
+    from tests.test_gpu_step_buffers import _same
+
+    print(f"restart of every slot donate={donate}", flush=True)
+    game = map_name_to_scenario("basesWorkers16x16", max_cycles=44)
+    b = game.bucket
+    env = nanorts_amd.make("NanoRTS", scenario=game, device="cuda:0")
+    _, state = env.reset(envmod.env_roots(3, 9))
+    env.rollout(state, 36, (5, 6), record=False)
+    state.core_state.leaves["time"][:4] = 43  # their next step is the horizon's
+    for name in ("hit_points", "carried_resources", "unit_type", "cell", "pending_issued_at"):
+        for first in (b.neutral_capacity + 40, b.neutral_capacity + b.per_player_capacity + 40):
+            state.core_state.leaves[name][:, first:first + 20] = 3
+    monkeypatch.setattr(envmod, "_FEW_GAMES", 0)
+    actions = env.sample_actions(env.get_avail_actions(state, form="words"), (7, 8), 0)
+    monkeypatch.setenv("NANORTS_AMD_FIRST_PASS", "lean")
+    want = env.step(None, state.clone(), actions, donate=donate)
+    monkeypatch.setenv("NANORTS_AMD_FIRST_PASS", "pair")
+    *_, taken = two_pass_step(env, state, actions)
+    assert set(taken.tolist()) == {1}
+    got = env.step(None, state.clone(), actions, donate=donate)
+    assert want[3]["__all__"].tolist() == [True] * 4 + [False] * 5
+    hp = want[1].core_state.leaves["hit_points"][:, b.neutral_capacity + 40]
+    assert hp.tolist() == [0] * 4 + [3] * 5
+    _same(want, got)
