@@ -9,8 +9,8 @@
 // each unit, candidate lists and the search scratch.  Decisions are per unit,
 // one lane per own slot; the walk over the queued units is sequential as in
 // the reference (each search sees the cells claimed before it); the searches'
-// straight paths run a lane each, the others one by one over LDS stacks, on
-// the lane of their unit (a lane per direction measured the same: 11.9 ms).
+// straight paths run a lane each, the others one by one over LDS stacks on
+// lane 0 (a lane per direction measured the same: 11.9 ms).
 #pragma once
 
 #include "engine.h"
@@ -943,10 +943,16 @@ NR_DEV int32_t translate_plan(const KGame& g, const Hdr& h, const Env& e, Bot& b
 // before up), and no cell nearer the target than the popped one has been
 // inserted yet.  So a search that reaches its range without a dead end walks
 // this path and answers its first step, with no stacks and no marks: only the
-// open cells are read.  `path` takes bit k set where step k is horizontal;
-// the answer is kSearch where the path meets a dead end (or is longer than
-// `path`), and the full search decides.  Start and goal are on the board and
-// the start is out of range.
+// open cells are read.  `path` takes bit k set where step k (of the first 64)
+// is horizontal; the answer is kSearch where the path meets a dead end, and the
+// full search decides.  Start and goal are on the board and the start is out of
+// range.
+// Paths past 64 steps are walked too: given up there, a unit that crosses a
+// large board paid for the walk and the full search both.  Seat rollouts of
+// 1024 games against WorkerRush on GardenOfWar64x64, 10 cycles: 10.0 ms with
+// full searches alone, 10.5 ms with paths given up at 64 steps and the full
+// searches on the units' lanes, 9.4 ms so ((2)Benzene, 128x112, 128 games:
+// 14.4, 16.0 and 13.9 ms).
 constexpr int32_t kSearch = 4, kStale = 5;  // beside the directions 0..3 and kAbsent
 NR_DEV int32_t straight_step(const KGame& g, const AS3 uint32_t* open, int32_t start, int32_t goal, int32_t range,
                              uint64_t* path, int32_t* length) {
@@ -959,13 +965,13 @@ NR_DEV int32_t straight_step(const KGame& g, const AS3 uint32_t* open, int32_t s
         if (dx * dx + dy * dy <= r2) break;
         const int32_t ch = cell + (dx < 0 ? -1 : 1), cv = cell + (dy > 0 ? W : -W);
         const bool oh = dx != 0 && bit_of(open, dx != 0 ? ch : cell), ov = dy != 0 && bit_of(open, dy != 0 ? cv : cell);
-        if ((!oh && !ov) || n == 64) {
+        if (!oh && !ov) {
             first = kSearch;
             break;
         }
         const bool h = oh && (!ov || across > along);
         if (n == 0) first = h ? across : along;
-        bits |= h ? 1ull << n : 0ull;
+        bits |= h && n < 64 ? 1ull << n : 0ull;
         ++n;
         cell = h ? ch : cv;
         if (h) dx += dx < 0 ? 1 : -1;
@@ -1074,9 +1080,14 @@ NR_DEV int32_t translate_walk(const KGame& g, const Hdr& h, const Env& e, Bot& b
                     for (int32_t c = lane; c < g.cells; c += TW) mark[c] = bit_of(open, c) ? 0 : 1;
                 }
                 wave_sync();
+                // (on lane 0 from operands that a whole wave holds in scalar
+                // registers: run on the unit's own lane from its registers,
+                // the search was 5 to 10 % slower and k_seat_rollout took 138
+                // VGPRs instead of 128)
                 int32_t s = kAbsent;
-                if (lane == q) s = astar_first_step(g, bv<int16_t>(b, y.a_below), mark, start, goal, radius);
-                now = tread_at<TW>(s, q);
+                const int32_t to = tread_at<TW>(goal, q), within = tread_at<TW>(radius, q);
+                if (lane == 0) s = astar_first_step(g, bv<int16_t>(b, y.a_below), mark, from, to, within);
+                now = tread_at<TW>(s, 0);
                 wave_sync();
             }
             const bool moves = now != kAbsent;
@@ -1092,13 +1103,15 @@ NR_DEV int32_t translate_walk(const KGame& g, const Hdr& h, const Env& e, Bot& b
                     open[claim >> 5] &= ~(1u << (claim & 31));
                     if (kept) claimed[claim >> 5] |= 1u << (claim & 31);
                 }
-                // a path through the cell: its step |ax| + |ay| lands there
+                // a path through the cell: its step |ax| + |ay| lands there (a
+                // step past the 64 that `path` holds may)
                 if (lane > q && step >= 0 && step < kSearch) {
                     const int32_t ax = cell_x(g, claim) - cell_x(g, start), ay = cell_y(g, claim) - cell_y(g, start);
                     const int32_t gx = cell_x(g, goal) - cell_x(g, start), gy = cell_y(g, goal) - cell_y(g, start);
                     const int32_t k = abs(ax) + abs(ay);
                     const uint64_t upto = k >= 64 ? ~0ull : (1ull << k) - 1ull;
-                    if (k <= length && ax * gx >= 0 && ay * gy >= 0 && __popcll(path & upto) == abs(ax)) step = kStale;
+                    if (k <= length && ax * gx >= 0 && ay * gy >= 0 && (k > 64 || __popcll(path & upto) == abs(ax)))
+                        step = kStale;
                 }
             }
             if (kept) {

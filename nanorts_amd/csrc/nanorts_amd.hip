@@ -2661,7 +2661,9 @@ NR_DEV void seat_cycles(const SeatRolloutArgs& args) {
 }
 
 // 168 VGPRs at most: three waves per SIMD, which the bot region's LDS allows
-// on boards up to 16x16
+// on boards up to 16x16 (it takes 128, so that four fit on smaller ones: 8192
+// games against WorkerRush on 10x10, 30 cycles, 2.37 ms at 138 VGPRs and
+// 1.97 ms at 128; bound to 128, GardenOfWar64x64 was 3 % slower)
 __global__ __launch_bounds__(256, 3) void k_seat_rollout(SeatRolloutArgs args) {
     (void)args;
     seat_cycles<false>(seat_args());

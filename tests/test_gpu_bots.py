@@ -291,3 +291,47 @@ def test_searches_on_crowded_boards(name):
         seat.rollout(sst, 24, (41, 43), record=False)
         assert_states_equal(ref, to_host(sst.environment_state), f"{name} fused")
         _assert_carry_equal(carry, _carry_to_host(sst.carry), f"{name} fused")
+
+
+@pytest.mark.parametrize("name", ["GardenOfWar64x64", "(4)BloodBath.scmA"])
+def test_searches_across_large_boards(name):
+    """Acts and seat cycles of units whose straight paths are longer than the
+    64 steps that the walk keeps of one: convoys from one corner to the other,
+    whose first cells close the paths of the units behind them, and crossings
+    past the sixty-fourth step."""
+    import torch
+
+    from nanorts_amd import bots
+    from nanorts_amd.bots import SeatState
+    from tests.test_gpu_parity import _packed
+
+    game = map_name_to_scenario(name, conflict_strategy=ConflictStrategy.CANCEL_BOTH, max_cycles=400)
+    o, b = Oracle(game), game.bucket
+    extra = [0, 3, 8, 20, 40, 80, 120, 160]
+    st = _packed(game, extra, seed=9)
+    assert (o.violations(st) == 0).all()
+    L, C = len(extra), b.per_player_capacity
+    cells = st["cell"][-1][st["birth"][-1] != -1].astype(int)
+    spread = np.abs(cells // b.width - cells[0] // b.width) + np.abs(cells % b.width - cells[0] % b.width)
+    assert spread.max() > 64
+    for bot in (WORKER_RUSH, BARRACKS_RUSH):
+        print(f"long searches {name} {bot}", flush=True)
+        seat = _seat_env(game, False, bot)
+        ref, carry = copy_state(st), empty_carry(L, C)
+        for t in range(24):
+            if t % 6 == 0:
+                for player in (0, 1):
+                    want_carry = copy_state(carry)
+                    want = o.abstraction_act(copy_state(ref), want_carry, bot, LIGHT, player)
+                    dev_carry = _carry_to_device(carry, seat.device)
+                    got = bots.abstraction_act(seat.env, to_device(seat.env, ref), dev_carry,
+                                               bots.Bot("probe", bot, LIGHT), player)
+                    for field, w in want.items():
+                        np.testing.assert_array_equal(got[field].cpu().numpy(), w, err_msg=f"{name} {t} {player} {field}")
+                    _assert_carry_equal(want_carry, _carry_to_host(dev_carry), f"{name} {t} {player}")
+            o.seat_step(ref, carry, bot, LIGHT, 0, _learner_actions(o, ref, t), False, observe=False)
+        sst = SeatState(to_device(seat.env, st), _carry_to_device(empty_carry(L, C), seat.device),
+                        torch.zeros(L, dtype=torch.int32, device=seat.device))
+        seat.rollout(sst, 24, (41, 43), record=False)
+        assert_states_equal(ref, to_host(sst.environment_state), f"{name} fused")
+        _assert_carry_equal(carry, _carry_to_host(sst.carry), f"{name} fused")
