@@ -1825,7 +1825,8 @@ NR_DEV Env team_env(const KGame& g, int team) {
 // 4096 games there, 50 cycles a launch, 2 % of them past 64 live slots: the
 // second pass took as long as the first (2.63 and 2.45 ms) while the first
 // held one slot a lane.
-template <bool Lean, int TW = kWave>
+// `Whole`: rows of whole observation groups (W % 4 == 0), as in summarize.
+template <bool Lean, int TW = kWave, bool Whole = Lean>
 NR_DEV void rollout_cycles(const RolloutArgs& args) {
     static_assert(TW == kWave || Lean, "half-wave teams run the first pass only");
     const KGame& g = args.g;
@@ -1870,7 +1871,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
     const bool fast = Lean || (g.fast_obs && ((((uintptr_t)args.out.feature_maps) & 7u) == 0));
     // the summary's counts stay in registers from one cycle into the next
     SlotSummary sm = {0, 0, 0, 0, false};
-    if (fast && fits) sm = summarize<TW, Lean, Lean>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
+    if (fast && fits) sm = summarize<TW, Lean, Whole>(g, hdr, e, lane, args.partial != 0, nullptr, nullptr, nullptr, nullptr);
     if (!fits) sm.full = true;
     uint32_t ek0 = (uint32_t)tuni<TW>(e.sc[S_ROOT0]), ek1 = (uint32_t)tuni<TW>(e.sc[S_ROOT1]);
     fold_in(ek0, ek1, (uint32_t)tuni<TW>(e.sc[S_EPISODE]));
@@ -2008,7 +2009,9 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
             }
             wave_sync();
             // env.step: core.step keyed by fold_in(env root, episode)
-            if (Lean || (fused && listed)) {
+            // (the weights keep the general admission's registers out of the
+            // cycle: without them the compiler spills around it everywhere)
+            if (__builtin_expect(Lean || (fused && listed), 1)) {
                 // the first pass stopped before any cycle that is not both
                 admit_resolve<TW>(g, hdr, e, lane, ek0, ek1, n, nA, posA, costA, playerA, q);
             } else if (fused || !admit_env(g, hdr, e, lane, ek0, ek1, false, n, irregular, true, fast)) {
@@ -2060,7 +2063,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
                 // the sight bitmaps persist in the event counters' words, which
                 // the rollout does not count, when both planes fit there
                 const int32_t kept = 2 * g.H * g.seen_words <= 32 ? g.lay.b_events : -1;
-                sm = summarize<TW, Lean, Lean>(g, hdr, e, lane, a.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr, kept);
+                sm = summarize<TW, Lean, Whole>(g, hdr, e, lane, a.partial != 0, m0, m0 ? m0 + per : nullptr, nullptr, nullptr, kept);
             } else if (out.feature_maps || out.scalars) {
                 observe_both(g, hdr, e, slot, lane, a.partial != 0, out.feature_maps, out.scalars);
             }
@@ -2081,7 +2084,13 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
     }
 }
 
-__global__ __launch_bounds__(256, 4) void k_rollout(RolloutArgs args) { rollout_cycles<false>(args); }
+// Boards whose rows are whole observation groups have a kernel without the other
+// boards' cell pass.  One pass over 8192 games on 16x16, 50 cycles, from 1.43 ms
+// before the general admission gave each request a lane and odd widths took the
+// summary, was 1.47 ms in one kernel for both without weights, 1.45 ms with them
+// and is 1.44 ms so.
+__global__ __launch_bounds__(256, 4) void k_rollout(RolloutArgs args) { rollout_cycles<false, kWave, true>(args); }
+__global__ __launch_bounds__(256, 4) void k_rollout_spanned(RolloutArgs args) { rollout_cycles<false>(args); }
 
 // The first pass: the one-wave path alone, on a smaller LDS block per game.
 // Without the request-by-request admission and completion's member records
@@ -4140,8 +4149,8 @@ int nanorts_amd_rollout(void* stream, const nanorts_game* game, nanorts_state st
             args.g = sh.g;
             args.resume = 1;
         }
-        hipLaunchKernelGGL(k_rollout, dim3((unsigned)blocks), dim3((unsigned)(kWave * sh.wpb)), (size_t)sh.lds,
-                           (hipStream_t)stream, args);
+        hipLaunchKernelGGL((sh.g.W & 3) == 0 ? k_rollout : k_rollout_spanned, dim3((unsigned)blocks),
+                           dim3((unsigned)(kWave * sh.wpb)), (size_t)sh.lds, (hipStream_t)stream, args);
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess)
             return fail(NANORTS_INTERNAL, std::string("kernel launch failed: ") + hipGetErrorString(err));
