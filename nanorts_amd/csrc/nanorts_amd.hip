@@ -424,6 +424,20 @@ bool shape_for_pair(const nanorts_game* game, Shape* out, bool any_occupancy, st
     return true;
 }
 
+// Whether games of a board outgrow any first pass of one game per wave:
+// nothing but the board bounds their units (a slot per cell), and it holds more
+// than the pass's 128 live slots and an eighth.  They leave it at some later
+// cycle, and a launch then takes the first pass's cycles and the full block's
+// one after the other.  There the window stays at 32 slots, and a launch of few
+// games keeps two games per wave, whose lower bounds send the crowded games to
+// the full block at once.  1024 games x 50 cycles on EightBasesWorkers16x12
+// 3.0 ms before either rule, 3.5 ms with 64 slots, one game per wave, and 2.1 ms
+// so; on EightBasesWorkers16x16 7.7, 5.6 and 4.5 ms; SixBasesWorkers12x12 (144
+// cells) is the other side of the line, 2.2 ms with 32 slots and 1.3 with 64.
+bool outgrows_first_pass(const nanorts_game* game) {
+    return game->capacity >= game->cells && game->cells > 128 + 128 / 8;
+}
+
 // The first pass's shape on the slot window (windowed): one game per wave
 // (shape_for_lean) or two (shape_for_pair).  The reset segments are the
 // window's business (reset_env's windowed path), so the table stays empty.
@@ -440,7 +454,8 @@ bool shape_for_first_pass(const nanorts_game* game, bool pair, bool any_occupanc
     // 3.34 -> 2.27 ms; FourBasesWorkers12x12: 32 -> 64 slots at 16 games, 1024
     // games x 100 cycles, a third of them handed over, 4.07 -> 2.03 ms;
     // TwoBasesBarracks16x16 2.98 -> 1.53 ms.
-    if (!pair && game->capacity >= 4 * kSlotWindow) {
+    // Not where the games outgrow that too (outgrows_first_pass).
+    if (!pair && game->capacity >= 4 * kSlotWindow && !outgrows_first_pass(game)) {
         const int32_t games = games_per_cu(out->g.lay, out->wpb, kLeanWavesPerSimd);
         for (int32_t slots = kSlotWindow + 8; shift > 0 && slots <= 2 * kSlotWindow; slots += 8) {
             Shape wider;
@@ -4080,7 +4095,8 @@ static int choose_first_pass(const nanorts_game* game, const Shape& full, int64_
         return 0;
     const ForcedPass forced = forced_first_pass();
     const bool want_pair = forced == ForcedPass::kPair;
-    if (forced == ForcedPass::kLean || (!want_pair && lanes > 0 && few_games(lanes, game->cells))) return 1;
+    const bool few = lanes > 0 && few_games(lanes, game->cells) && !outgrows_first_pass(game);
+    if (forced == ForcedPass::kLean || (!want_pair && few)) return 1;
     return shape_for_first_pass(game, true, want_pair, pair, &why) ? 2 : 1;
 }
 

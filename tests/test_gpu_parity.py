@@ -534,6 +534,36 @@ def test_lean_first_pass_holds_two_live_slots_a_lane(monkeypatch, oracle_threads
     assert_states_equal(st, to_host(dev), "lean pass, two live slots a lane")
 
 
+@pytest.mark.parametrize("name,wide", [("EightBasesWorkers16x12", False), ("EightBasesWorkers16x16", False),
+                                       ("SixBasesWorkers12x12", True), ("TwoBasesBarracks16x16", True)])
+def test_lean_window_by_board(name, wide, monkeypatch, oracle_threads):
+    """One game per wave on boards of 128 or more slots a player: a game whose
+    players hold 33 to 44 slots runs in the first pass where its window is the
+    wide one, and in the second from its first cycle where nothing but a board
+    of many cells bounds the units, whose window is 32 slots."""
+    from nanorts_amd.content import map_name_to_scenario
+    from oracle.oracle import Oracle
+
+    _first_pass(monkeypatch, "lean")
+    print("lean window", name, flush=True)
+    game = map_name_to_scenario(name, max_cycles=300, conflict_strategy="CANCEL_RANDOM")
+    b = game.bucket
+    own = int((_packed(game, [0])["birth"][0, b.neutral_capacity:b.neutral_capacity + b.per_player_capacity] != -1).sum())
+    st = _packed(game, [n - own for n in (20, 28, 33, 36, 40, 44)], alternate=False)
+    oracle = Oracle(game)
+    assert (oracle.violations(st) == 0).all()
+    env = _env(game, True)
+    dev = to_device(env, st)
+    got = env.rollout(dev, 12, (1, 2), record=True)
+    want = oracle.rollout(st, (1, 2), 0, 12, True, threads=oracle_threads)
+    first = got["first_pass_cycles"].cpu().numpy()
+    print("first-pass cycles per game:", first.tolist(), flush=True)
+    assert first[0] > 0 and ((first[2:] > 0).all() if wide else (first[2:] == 0).all())
+    np.testing.assert_array_equal(got["rewards"].cpu().numpy(), want["rewards"])
+    np.testing.assert_array_equal(got["feature_maps"][0].cpu().numpy(), want["feature_maps"])
+    assert_states_equal(st, to_host(dev), name)
+
+
 def test_crowded_env_step_per_call(oracle_threads):
     """env.step on the same crowded states, cycle by cycle, against the oracle."""
     import torch
