@@ -400,16 +400,17 @@ nanorts_game windowed(const nanorts_game* game, int32_t* shift, int32_t slots = 
 // shape whatever it fits.
 constexpr int kPairMaxWaves = 4;
 constexpr int kPairMinGamesPerCu = 2 * 3 * 4;
+int32_t pair_games_per_cu(const Layout& y, int w) {
+    const int32_t by_lds = lds_per_cu() / lds_granule(y.hdr_bytes + 2 * w * y.env_bytes);
+    const int32_t by_waves = (4 * kLeanWavesPerSimd) / w;
+    return (by_lds < by_waves ? by_lds : by_waves) * 2 * w;
+}
 bool shape_for_pair(const nanorts_game* game, Shape* out, bool any_occupancy, std::string* why) {
     if (!shape_for_lean(game, out, why)) return false;
     const Layout& y = out->g.lay;
     int best = 0, best_w = 0;
     for (int w = 1; w <= kPairMaxWaves; ++w) {
-        const int32_t bytes = y.hdr_bytes + 2 * w * y.env_bytes;
-        if (bytes > lds_per_cu()) continue;
-        const int32_t by_lds = lds_per_cu() / lds_granule(bytes);
-        const int32_t by_waves = (4 * kLeanWavesPerSimd) / w;
-        const int games = (by_lds < by_waves ? by_lds : by_waves) * 2 * w;
+        const int games = pair_games_per_cu(y, w);
         if (games > best) {
             best = games;
             best_w = w;
@@ -474,6 +475,15 @@ bool shape_for_first_pass(const nanorts_game* game, bool pair, bool any_occupanc
 }
 
 
+// Compute units of the current device; 0 where there is none.
+int32_t compute_units() {
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return 0;
+    return cus;
+}
+
 // Whether a launch has so few games that one game per wave is the faster
 // first pass: a wave of two games pays by issuing less, but each of its cycles
 // takes longer, and with few waves a SIMD it is the length of a cycle that
@@ -485,11 +495,38 @@ bool shape_for_first_pass(const nanorts_game* game, bool pair, bool any_occupanc
 // 2.61 / 1.62 (2048), 2.72 / 2.07 (4096); 8x8 0.88 / 0.81 (1024), 0.91 / 0.89
 // (2048), 0.98 / 1.14 (4096).
 bool few_games(int64_t lanes, int32_t cells) {
-    int device = 0, cus = 0;
-    if (hipGetDevice(&device) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0)
-        return false;
-    return lanes <= (int64_t)(cells >= 4 * kWave ? 16 : 8) * cus;
+    return lanes <= (int64_t)(cells >= 4 * kWave ? 16 : 8) * compute_units();
+}
+
+// Whether env.step of so many games is faster as two launches (k_env_step_pair,
+// then k_env_step for the games it leaves) than as one: by the rounds of games
+// that the full block takes, at k_env_step's seven waves a SIMD.  The second
+// launch costs 8 us of host time and, where it has a game to step, the length of
+// a step of its own, so the first has to save rounds:
+// - fewer than 128 slots a player, whose games stay in the window: from two
+//   rounds, or from 7/6 where the first pass holds more than twice the games.
+//   A masks-sample-step turn with one launch against two, on its own / among
+//   others, us: 16x16 (16 and 32 games a CU) 1.5 rounds 133 / 131, 91 / 100, two
+//   143 / 137, 102 / 99; 8x8 (24 and 32) 1.3 rounds 132 / 123, 89 / 98, 2.3
+//   158 / 147, 126 / 112; 12x12 (12 and 32) one round 125 / 124, 90 / 99, 7/6
+//   156 / 127, 109 / 98; 24x24 (8 and 28) one 130 / 133, 93 / 101, 1.5 169 / 138,
+//   125 / 101.
+// - 128 or more, where games outgrow the window: past two rounds and 16 games a
+//   CU.  TwoBasesBarracks16x16 (8 and 32) two rounds 160 / 176, 116 / 128, one
+//   game more 191 / 177, 147 / 132; DoubleGame24x24 (4 and 24) two 254 / 302,
+//   222 / 267, four 413 / 404, 391 / 382.
+// - a slot per cell there: most games are past it, so from eight rounds, and
+//   where neutral units leave the players three quarters of its 64 live slots.
+//   FourBasesWorkers12x12 (8 and 32, 14 neutral units) six rounds 431 / 443,
+//   408 / 419, eight 605 / 572, 585 / 553; SixBasesWorkers12x12 (22) two rounds
+//   202 / 252, eight 666 / 730, sixteen 1321 / 1444.
+bool two_launches_pay(int64_t lanes, const nanorts_game* game, const Shape& full, bool* most) {
+    const int64_t resident = (int64_t)games_per_cu(full.g.lay, full.wpb, 7) * compute_units();
+    *most = lanes >= 2 * resident;  // whatever the first pass holds
+    if (resident <= 0) return false;
+    if (game->capacity < 4 * kSlotWindow) return 6 * lanes >= 7 * resident;
+    if (game->capacity >= game->cells) return game->neutral <= kWave / 4 && lanes >= 8 * resident;
+    return lanes > 2 * resident && lanes > 16 * (int64_t)compute_units();
 }
 
 // The first pass that the environment variable NANORTS_AMD_FIRST_PASS asks
@@ -2132,10 +2169,9 @@ __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_rollout_pair(Rollo
 // only).  A game that does not fit (a state or an initial state outside the
 // window, an irregular state, more than 32 available units or 64 live slots, a
 // spawn that could land past the window) is left untouched for k_env_step,
-// with taken[l] = 0.  65536 games on 16x16 in place: 471 us in k_env_step,
-// 375 us in both.  Few games run in k_env_step alone: with at most one
-// game per wave a SIMD the length of one step counts, not the waves in flight
-// (few_games' line; a second launch would cost 4 us more).
+// with taken[l] = 0.  A masks-sample-step turn of 65536 games on 16x16 takes
+// 650 us with k_env_step alone and 567 us with both; two_launches_pay has the
+// other sizes.
 struct EnvStepArgs {
     KGame g;  // first: fresh_game() reads it at offset 0
     int64_t lanes;
@@ -3701,10 +3737,13 @@ static int env_step(void* stream, const nanorts_game* game, const nanorts_state&
     Shape pair;
     std::string why;
     const ForcedPass forced = forced_first_pass();
+    const bool asked = forced == ForcedPass::kPair;
+    bool most = false;
     const bool paired = taken && lanes > 0 && forced != ForcedPass::kLean &&
-                        (forced == ForcedPass::kPair || !few_games(lanes, game->cells)) &&
+                        (asked || two_launches_pay(lanes, game, sh, &most)) &&
                         ((((uintptr_t)results.feature_maps) | ((uintptr_t)results.final_feature_maps)) & 7u) == 0 &&
-                        shape_for_first_pass(game, true, forced == ForcedPass::kPair, &pair, &why);
+                        shape_for_first_pass(game, true, asked, &pair, &why) &&
+                        (asked || most || pair_games_per_cu(pair.g.lay, pair.wpb) > 2 * games_per_cu(sh.g.lay, sh.wpb, 7));
     if (paired) {
         EnvStepArgs args;
         std::memset(&args, 0, sizeof(args));

@@ -128,7 +128,7 @@ def test_env_step_reads_actions_where_they_lie(name, L):
     _same(env.step(None, state, same_everywhere), env.step(None, state, expanded))
 
 
-@pytest.mark.parametrize("name,L,partial", [("basesWorkers8x8", 2051, False), ("basesWorkers16x16", 4099, True),
+@pytest.mark.parametrize("name,L,partial", [("basesWorkers8x8", 12803, False), ("basesWorkers16x16", 8707, True),
                                             ("basesWorkers32x32A", 4098, True)])
 def test_env_step_of_many_games_in_two_passes(name, L, partial, monkeypatch):
     """More games than one pass takes: the launch of two games per wave and the

@@ -159,3 +159,31 @@ def test_restart_replaces_every_slot(donate, monkeypatch):
     hp = want[1].core_state.leaves["hit_points"][:, b.neutral_capacity + 40]
     assert hp.tolist() == [0] * 4 + [3] * 5
     _same(want, got)
+
+
+# games per compute unit on either side of the line between one launch and two
+# (None: one launch however many)
+@pytest.mark.parametrize("name,one,two", [
+    ("basesWorkers8x8", 46, 50), ("basesWorkers16x16", 30, 34), ("basesWorkers12x12", 13, 15),
+    ("basesWorkers32x32A", 8, 11), ("TwoBasesBarracks16x16", 16, 18), ("SixBasesWorkers12x12", 66, None),
+    ("FourBasesWorkers12x12", 60, 66),
+    ("GardenOfWar64x64", 8, None)])
+def test_launches_by_board_and_games(name, one, two, monkeypatch):
+    """env.step of few games is one launch and of many two, by the board: the
+    work words are left alone in the one and written in the other."""
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import env as envmod
+
+    monkeypatch.delenv("NANORTS_AMD_FIRST_PASS", raising=False)
+    env = nanorts_amd.make("NanoRTS", scenario=map_name_to_scenario(name), device="cuda:0", final_observation=True)
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    for games in (one, two):
+        if games is None:
+            continue
+        print(f"launches {name} {games} games a unit", flush=True)
+        _, state = env.reset(envmod.env_roots(3, games * units))
+        actions = env.sample_actions(env.get_avail_actions(state, form="words"), (7, 8), 0)
+        *_, taken = two_pass_step(env, state, actions)
+        assert set(taken.tolist()) == ({UNTOUCHED} if games == one else {1})
