@@ -31,12 +31,16 @@ CASES = {
     # attack window next to the range-1 neighbour masks
     "ranged-random": ("melee8x8Mixed6", UnitTypeTableVersion.ORIGINAL_FINETUNED, ConflictStrategy.CANCEL_RANDOM, 300,
                       True, True),
-    # widths that are not a multiple of 4: the kernels' general observation
-    # and summary branches
+    # widths that are not a multiple of 4: observation groups that span two
+    # rows
     "10x10-random-partial": ("basesWorkers10x10", UnitTypeTableVersion.ORIGINAL_FINETUNED,
                              ConflictStrategy.CANCEL_RANDOM, 5000, True, True),
     "9x8-alternating": ("NoWhereToRun9x8", UnitTypeTableVersion.ORIGINAL, ConflictStrategy.CANCEL_ALTERNATING, 130,
                         True, False),
+    # a cell count that is not a multiple of 4 either: the kernels' general
+    # branches (cell-by-cell observation, masks from the grid, no summary)
+    "15x14-random-partial": ("itsNotSafe", UnitTypeTableVersion.ORIGINAL, ConflictStrategy.CANCEL_RANDOM, 140, True,
+                             True),
     # boards 17-32 wide: the 32-bit row masks of the visibility and window
     # passes, with walls (barricades) and partial observability
     "24x24-barricades-alternating": ("barricades24x24", UnitTypeTableVersion.ORIGINAL_FINETUNED,

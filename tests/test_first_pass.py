@@ -26,7 +26,7 @@ def _first_pass(case: str) -> int:
 @pytest.mark.parametrize("case, want", [
     ("16x16-random-partial", 2), ("16x16-noprofile-random", 2), ("8x8-original-both", 2), ("melee-both", 2),
     ("24x24-barricades-alternating", 2), ("32x32-random-partial", 2), ("gow-alternating", 1),
-    ("10x10-random-partial", 0), ("9x8-alternating", 0),
+    ("10x10-random-partial", 0), ("9x8-alternating", 0), ("15x14-random-partial", 0),
 ])
 def test_first_pass_by_board(case, want, monkeypatch):
     monkeypatch.delenv("NANORTS_AMD_FIRST_PASS", raising=False)

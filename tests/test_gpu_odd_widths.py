@@ -1,5 +1,6 @@
 """Boards whose width is not a multiple of 4: the summary's observation groups
-of four cells span two rows there.  Every observation, mask, fused rollout and
+of four cells span two rows there, or there is no summary where the cells are
+no multiple of 4 (15x14).  Every observation, mask, fused rollout and
 seat rollout against the oracle, bit for bit, with and without hidden
 information; walls, both orders of an observation's rows and units on every
 column come with the boards' random play."""
@@ -15,7 +16,7 @@ from tests.helpers import assert_states_equal, roots, to_device, to_host
 
 pytestmark = pytest.mark.gpu
 
-BOARDS = ("NoWhereToRun9x8", "basesWorkers10x10", "melee14x12Mixed18")
+BOARDS = ("NoWhereToRun9x8", "basesWorkers10x10", "itsNotSafe", "melee14x12Mixed18")
 
 
 def _env(game, partial, **kw):
@@ -62,7 +63,7 @@ def test_steps_and_rollouts_match_oracle(name, partial, oracle_threads):
 
 
 @pytest.mark.parametrize("partial", [False, True])
-@pytest.mark.parametrize("name", BOARDS[:2])
+@pytest.mark.parametrize("name", BOARDS[:3])
 def test_seat_rollouts_match_oracle(name, partial):
     import torch
 

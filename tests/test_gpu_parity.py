@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
 
 FAST_CASES = ["8x8-original-both", "16x16-finetuned-both", "16x16-random-partial", "16x16-alternating",
               "melee-both", "barracks-random", "obstacle-alternating", "10x10-random-partial", "9x8-alternating",
+              "15x14-random-partial",
               "ranged-random", "24x24-barricades-alternating", "32x32-random-partial"]
 
 
@@ -137,8 +138,9 @@ def _poison_allocator(nbytes: int) -> None:
 
 
 def _first_pass(monkeypatch, mode: str) -> None:
-    """Select the rollout's first pass: "auto" (the library's choice by
-    board), "lean" (one game per wave) or "pair" (two games per wave)."""
+    """Select the rollout's first pass: "auto" (the library's choice by board
+    and games: for the few of these tests one game per wave, or none), "lean"
+    (one game per wave) or "pair" (two games per wave)."""
     if mode == "auto":
         monkeypatch.delenv("NANORTS_AMD_FIRST_PASS", raising=False)
     else:
@@ -151,7 +153,8 @@ def _first_pass(monkeypatch, mode: str) -> None:
 def test_fused_rollout_matches_oracle(case, recorded, first_pass, monkeypatch, oracle_threads):
     """The fused rollout kernel over a long horizon against the oracle's
     rollout: per-cycle rewards and dones, the recorded actions, last
-    observation and the final state, with each first pass.  Unrecorded, the
+    observation and the final state, with each first pass and with the
+    library's own choice for so few games.  Unrecorded, the
     kernel draws only the factors its decode reads; the game must not
     change."""
     _first_pass(monkeypatch, first_pass)
@@ -420,21 +423,22 @@ def test_two_pass_rollout_hands_games_to_the_second_pass(first_pass, monkeypatch
     assert_states_equal(st, to_host(one), "one-pass rollout")
 
 
-@pytest.mark.parametrize("first_pass", ["auto", "pair"])
-def test_pair_first_pass_hands_games_to_the_second_pass(first_pass, monkeypatch, oracle_threads):
-    """With two games per wave (the choice on 8x8 boards) the first pass runs
-    a game while it has at most 32 available units, 64 live slots and room
-    in its slot window; the second pass runs the rest.  Games that start with
+@pytest.mark.parametrize("first_pass", ["lean", "pair"])
+def test_first_pass_hands_games_of_an_8x8_board_to_the_second_pass(first_pass, monkeypatch, oracle_threads):
+    """With two games per wave the first pass runs a game while it has at most
+    32 available units, 64 live slots and room in its slot window, with one
+    game per wave while it has at most 64, 128 and that room; the second pass
+    runs the rest.  Games that start with
     24..40 live slots on basesWorkers8x8, the added Workers all player 0's
     and 200 resources each, cross a bound at cycle 0 or not at all (on this
     crowded board no spawn takes a game past its window within the launch;
     the 16x16 test above crosses part-way).  All of them match the oracle;
-    an odd number of games leaves the last wave's second half without a
-    game."""
+    an odd number of games leaves the last wave's second half (the last
+    workgroup's last waves) without a game."""
     from oracle.oracle import Oracle
 
     _first_pass(monkeypatch, first_pass)
-    print("pair two-pass rollout", flush=True)
+    print("8x8 two-pass rollout", first_pass, flush=True)
     game, partial = game_for("8x8-original-both")
     base = int((_packed(game, [0])["birth"][0] != -1).sum())
     extra = [24 - base + k for k in range(17)]
@@ -460,11 +464,12 @@ def test_pair_first_pass_hands_games_to_the_second_pass(first_pass, monkeypatch,
     assert_states_equal(st, to_host(dev), "pair two-pass rollout")
 
 
-@pytest.mark.parametrize("first_pass", ["auto", "pair"])
-def test_pair_first_pass_holds_two_live_slots_and_two_entries_a_lane(first_pass, monkeypatch, oracle_threads):
-    """Two games per wave with 33..64 live slots and 33..64 pending MOVE /
-    PRODUCE entries per game: each lane of a half-wave team holds two of
-    each (completion's members, admission's claims).  Crowded 16x16 games
+@pytest.mark.parametrize("first_pass", ["lean", "pair"])
+def test_first_pass_holds_33_to_64_live_slots_and_entries(first_pass, monkeypatch, oracle_threads):
+    """33..64 live slots and 33..64 pending MOVE / PRODUCE entries per game:
+    with two games per wave each lane of a half-wave team holds two of each
+    (completion's members, admission's claims), with one game per wave one.
+    Crowded 16x16 games
     (44..51 live slots, Workers of both players), advanced 12 cycles by the
     oracle so that most units hold a pending action, stay in the first pass
     for the whole launch, reach more than 32 entries, and match the
@@ -472,7 +477,7 @@ def test_pair_first_pass_holds_two_live_slots_and_two_entries_a_lane(first_pass,
     from oracle.oracle import Oracle
 
     _first_pass(monkeypatch, first_pass)
-    print("pair pass, crowded", first_pass, flush=True)
+    print("first pass, crowded", first_pass, flush=True)
     game, partial = game_for("16x16-random-partial")
     b = game.bucket
     base = int((_packed(game, [0])["birth"][0] != -1).sum())
@@ -532,6 +537,37 @@ def test_lean_first_pass_holds_two_live_slots_a_lane(monkeypatch, oracle_threads
     np.testing.assert_array_equal(got["feature_maps"][0].cpu().numpy(), want["feature_maps"])
     np.testing.assert_array_equal(got["scalars"][0].cpu().numpy(), want["scalars"])
     assert_states_equal(st, to_host(dev), "lean pass, two live slots a lane")
+
+
+@pytest.mark.parametrize("name,crowd,per_unit", [("basesWorkers8x8", 20, 8), ("basesWorkers16x16", 20, 16),
+                                                  ("EightBasesWorkers16x12", 18, 0)])
+def test_few_games_run_one_game_per_wave(name, crowd, per_unit, monkeypatch):
+    """The library's choice by the number of games, on either side of its line
+    (8 or 16 games a compute unit): its first game, with 33..64 available units
+    or more than 64 live slots, runs in the pass of one game per wave and not in
+    that of two.  A board whose games outgrow the former takes the latter
+    however few they are."""
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import env as envmod
+    from nanorts_amd.content import map_name_to_scenario
+
+    _first_pass(monkeypatch, "auto")
+    game = map_name_to_scenario(name)
+    b = game.bucket
+    own = [int((_packed(game, [0])["birth"][0, b.neutral_capacity + p * b.per_player_capacity:][:b.per_player_capacity]
+                != -1).sum()) for p in (0, 1)]
+    crowded = to_device(_env(game, False), _packed(game, [2 * crowd - sum(own)]))
+    env = nanorts_amd.make("NanoRTS", scenario=game)
+    line = per_unit * torch.cuda.get_device_properties(0).multi_processor_count
+    for games, first in ((line or 64, 2 if line else 0), (line + 1 if line else 256, 0)):
+        print(f"few games {name} {games}", flush=True)
+        _, state = env.reset(envmod.env_roots(3, games))
+        for k, v in crowded.core_state.leaves.items():
+            state.core_state.leaves[k][:1] = v
+        out = env.rollout(state, 2, (1, 2), record=False)
+        assert out["first_pass_cycles"].tolist() == [first] + [2] * (games - 1)
 
 
 @pytest.mark.parametrize("name,wide", [("EightBasesWorkers16x12", False), ("EightBasesWorkers16x16", False),
