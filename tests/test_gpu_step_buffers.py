@@ -2,8 +2,8 @@
 state and writes another.  Each step surface is compared with itself on a
 donated copy (which the other tests compare with the oracle), bit for bit,
 and the input state must stay as it was.  The boards cover both row copies
-(whole vectors and by granule), both observation branches and a state with a
-strided leaf, which is copied first.  Horizons are short, so games end and
+(whole vectors and by granule), the summary's observation and the general one
+(15x14) and a state with a strided leaf, which is copied first.  Horizons are short, so games end and
 reset inside the steps."""
 from __future__ import annotations
 
@@ -17,7 +17,8 @@ from nanorts_amd.content import map_name_to_scenario
 pytestmark = pytest.mark.gpu
 
 # map, games (odd counts leave the last workgroup short)
-BOARDS = (("basesWorkers8x8", 65), ("NoWhereToRun9x8", 33), ("basesWorkers16x16", 66), ("basesWorkers24x24A", 5))
+BOARDS = (("basesWorkers8x8", 65), ("NoWhereToRun9x8", 33), ("itsNotSafe", 33), ("basesWorkers16x16", 66),
+          ("basesWorkers24x24A", 5))
 
 
 def _say(*parts):
@@ -173,7 +174,7 @@ def test_env_step_of_many_games_in_two_passes(name, L, partial, monkeypatch):
     assert seen == {0, 1} and ends > 0  # both launches stepped games
 
 
-@pytest.mark.parametrize("name,L", BOARDS[:3])
+@pytest.mark.parametrize("name,L", BOARDS[:4])
 @pytest.mark.parametrize("rule", ["player_1", "drawn"])
 def test_seat_step_writes_fresh_buffers(name, L, rule):
     import torch
@@ -245,3 +246,103 @@ def test_step_from_entries_refuse_bad_arguments():
     code = lib.nanorts_amd_seat_step_from(None, dev.ref, whole, whole, 1, 0, 4, 0, addr, None, 1, carry, carry, addr, 0,
                                           native.EnvResults())
     assert code == 1 and "seats" in lib.nanorts_amd_last_error().decode()
+
+
+@pytest.mark.parametrize("name,L", BOARDS[:3])
+def test_in_place_entries_match_the_from_entries(name, L):
+    """The C entries that step a state in place (the facades call the ones with
+    a state of their own to write) on stacked action rows of both agents:
+    outputs and state as the facades' steps have them."""
+    import torch
+
+    import nanorts_amd
+    from nanorts_amd import bots, gridnet, native
+    from nanorts_amd import env as envmod
+
+    _say(f"in-place entries {name}")
+    lib, stream = native.load(), torch.cuda.current_stream().cuda_stream
+    game = map_name_to_scenario(name, max_cycles=34, conflict_strategy="CANCEL_ALTERNATING")
+    env = nanorts_amd.make("NanoRTS", scenario=game, partial_observability=True, reward_components=True,
+                           device="cuda:0")
+    b = env.bucket
+    _, state = env.reset(envmod.env_roots(3, L))
+    env.rollout(state, 30, (5, 6), record=False)
+
+    def buffers(final):
+        _poison()
+        maps, flags = (L, 2, b.height, b.width, 6), {"dtype": torch.bool, "device": "cuda:0"}
+        out = {"reward": torch.empty((L, 2), device="cuda:0"), "done": torch.empty(L, **flags),
+               "terminated": torch.empty(L, **flags), "truncated": torch.empty(L, **flags),
+               "winner": torch.empty(L, dtype=torch.int32, device="cuda:0"),
+               "spawn_overflowed": torch.empty(L, **flags), "maps": torch.empty(maps, dtype=torch.uint8, device="cuda:0"),
+               "scalars": torch.empty((L, 2, 4), dtype=torch.int32, device="cuda:0"), "final_maps": None,
+               "final_scalars": None, "components": None, "spawn_overflow": None}
+        if final:
+            out["final_maps"], out["final_scalars"] = torch.empty_like(out["maps"]), torch.empty_like(out["scalars"])
+        return out, native.EnvResults(*[None if t is None else t.data_ptr() for t in out.values()])
+
+    def check(got, nxt, want, agents=None):
+        obs, state_, rewards, dones, infos = want
+        _same(state_, nxt)
+        assert torch.equal(got["done"], dones["__all__"])
+        for name_ in ("terminated", "truncated", "winner", "spawn_overflowed"):
+            assert torch.equal(got[name_], infos[name_]), name_
+        for p, agent in enumerate(agents or ()):
+            assert torch.equal(got["reward"][:, p], rewards[agent])
+            assert torch.equal(got["maps"][:, p], obs[agent].feature_maps)
+            assert torch.equal(got["scalars"][:, p], obs[agent].scalars)
+            if got["final_maps"] is not None:
+                assert torch.equal(got["final_maps"][:, p], infos["final_observation"][agent].feature_maps)
+
+    seat = bots.SeatEnv(bots.workerRushAI, scenario=game, seat="drawn", device="cuda:0")
+    _, sst = seat.reset(envmod.env_roots(4, L))
+    seat.rollout(sst, 30, (5, 6), record=False)
+    grid = gridnet.GridNet(game, gridnet.prepare(game, mask_form="packed"), device="cuda:0")
+    ends = 0
+    for t in range(8):
+        words = env.get_avail_actions(state, form="words")
+        actions = env.sample_actions(words, (7, 8), t)
+        rows = torch.stack([actions[a] for a in env.agents], dim=1).contiguous()
+        for entry, step, final in ((lib.nanorts_amd_env_transition, env.step_env, False),
+                                   (lib.nanorts_amd_env_step, env.step, True)):
+            want, nxt = step(None, state, actions), state.clone()
+            got, results = buffers(final)
+            native.check(entry(stream, env.dev.ref, nxt.native(), L, rows.data_ptr(), env.partial, results), "in place")
+            check(got, nxt, want, env.agents)
+        ends += int(want[3]["__all__"].sum())
+        state = want[1]
+
+        learner = {bots.LEARNER: torch.where(sst.seat.reshape(-1, 1, 1) == 0, *[actions[a] for a in env.agents]).contiguous()}
+        want, nxt = seat.step(None, sst, learner), sst.clone()
+        got, results = buffers(False)
+        es = nxt.environment_state
+        native.check(lib.nanorts_amd_seat_step_lanes(
+            stream, seat.env.dev.ref, es.native(), L, seat.bot.strategy, seat.bot.trained, nxt.seat.data_ptr(), 1,
+            bots._carry_struct(nxt.carry), learner[bots.LEARNER].data_ptr(), seat.env.partial, results), "seat in place")
+        check(got, nxt, want)
+        nxt = sst.clone()
+        nxt.seat[:] = 1
+        fixed, results = buffers(False)
+        native.check(lib.nanorts_amd_seat_step(
+            stream, seat.env.dev.ref, nxt.environment_state.native(), L, seat.bot.strategy, seat.bot.trained, 1,
+            bots._carry_struct(nxt.carry), learner[bots.LEARNER].data_ptr(), seat.env.partial, results), "seat in place")
+        second = (sst.seat == 1).nonzero().reshape(-1)
+        for field in ("reward", "done", "winner", "maps", "scalars"):
+            assert torch.equal(fixed[field][second], got[field][second]), field
+        sst = want[1]
+
+        cells = grid.sample_actions(grid.observe(state).action_mask, (1, 2), t)
+        commands = grid.decode_actions(cells, state)
+        first = cells[:, 0].contiguous()
+        for entry, step, drawn, extra in (
+                (lib.nanorts_amd_gridnet_step, lambda s: grid.step(s, cells), cells, ()),
+                (lib.nanorts_amd_gridnet_step_against, lambda s: grid.step_against(s, first, commands), first,
+                 (native.Commands(*[commands[f].data_ptr() for f, _ in native.Commands._fields_]),))):
+            want, nxt = step(state), state.clone()
+            done = torch.empty(L, dtype=torch.bool, device="cuda:0")
+            comps = torch.empty_like(want.reward_components)
+            results = native.GridNetResults(comps.data_ptr(), None, None, None, done.data_ptr())
+            native.check(entry(stream, grid.dev.ref, nxt.native(), L, drawn.data_ptr(), *extra, results), "grid in place")
+            _same(want.environment_state, nxt)
+            assert torch.equal(done, want.done) and torch.equal(comps, want.reward_components)
+    assert ends > 0
