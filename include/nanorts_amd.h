@@ -154,15 +154,16 @@ typedef struct nanorts_rollout_results {
     uint8_t* feature_maps;  /* [depth][L][2][H][W][6]; step t writes slot t % depth */
     int32_t* scalars;       /* [depth][L][2][4] */
     int32_t depth;          /* ring depth of feature_maps / scalars, >= 1 */
-    int32_t* general_admissions; /* [L] cycles of the launch admitted request by request (an irregular
+    int32_t* general_admissions; /* [L] cycles of the launch that took the general admission (an irregular
                                   * state or more than 64 requests); written by nanorts_amd_rollout only */
-    int32_t* progress;           /* [L] caller-owned work words of nanorts_amd_rollout's two-pass launch, or
-                                  * NULL for one pass on the full LDS block.  With them, a first pass runs
+    int32_t* progress;           /* [L] caller-owned work words of the rollouts' two-pass launch, or NULL
+                                  * for one pass on the full LDS block.  With them, a first pass runs
                                   * each game on a smaller LDS block (more games per CU) until a cycle needs
-                                  * the request-by-request admission or more than 64 live slots complete;
-                                  * the second pass runs the rest of that game's cycles on the full block.
-                                  * On return: the cycles of the last launch each game ran in the first
-                                  * pass.  Ignored by the seat rollouts. */
+                                  * the general admission, more live slots or available units than its
+                                  * lanes hold (128 and 64 with one game per wave, 64 and 32 with two) or
+                                  * slots past its window; the second pass runs the rest of that game's
+                                  * cycles on the full block.  On return: the cycles of the last launch
+                                  * each game ran in the first pass. */
 } nanorts_rollout_results;
 
 /* Carry of an abstraction-family bot (AbstractActions,
@@ -464,7 +465,8 @@ int nanorts_amd_rollout(void* stream, const nanorts_game* game, nanorts_state st
  * aligned or absent) of games that fill the device: 2 two games per wave, 1
  * one game per wave, 0 none (one pass on the full block); < 0 an error code.
  * A launch of few games (at most 16 per compute unit, 8 on boards below 256
- * cells) runs 1 where this says 2.  Diagnostics only: it has no
+ * cells) runs 1 where this says 2, except on boards of more than 144 cells
+ * with a slot per cell for each player.  Diagnostics only: it has no
  * counterpart in the reference, whose program has no such launch. */
 int nanorts_amd_rollout_first_pass(const nanorts_game* game);
 

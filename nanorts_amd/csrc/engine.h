@@ -776,7 +776,7 @@ NR_DEV bool load_window_rows(const KGame& g, const nanorts_state& s, int64_t l, 
     // kSets slots a lane at a time: every leaf's load of every set first, then
     // the LDS stores, so that a kernel's first load waits on memory once for
     // kWindowSets * TW slots (one set at a time, a step of 65536 games on 16x16,
-    // 68 slots on 32 lanes, took 360 us instead of 326 us); a reset
+    // 68 slots on 32 lanes, took 360 us instead of 325 us); a reset
     // inside a kernel, where registers are short, takes one set
     for (int32_t base = 0; base < E; base += kSets * TW) {
 #define NR_DECLARE(flag, field, member, type, count) type v_##member[kSets];

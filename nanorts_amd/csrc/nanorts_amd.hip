@@ -314,11 +314,11 @@ int32_t games_per_cu(const Layout& y, int wpb, int waves_per_simd) {
 // one-wave path uses: the summary's bitmaps and lists that persist into the
 // next cycle's sampling and admission, and the summary's temporaries.  A
 // cycle that would need more (an irregular state,
-// more than 64 available units or 128 live slots) is left to the second pass,
-// on the full block.  The command arrays, the request-by-request
-// admission's keys, completion's member records and the staging of the
-// non-packed observation have no place in this block and are never used
-// by k_rollout_lean.  The entry list keeps 64 entries: the summary writes no
+// more than 64 available units or 128 live slots; half as many with two games
+// per wave) is left to the second pass, on the full block.  The command arrays,
+// the general admission's keys, completion's member records and the staging
+// of the non-packed observation have no place in this block and are never
+// used by the first passes.  The entry list keeps 64 entries: the summary writes no
 // more, and more than 64 entries is an irregular state.
 bool shape_for_lean(const nanorts_game* game, Shape* out, std::string* why) {
     if (!shape_for(game, out, why)) return false;
@@ -368,7 +368,8 @@ bool shape_for_lean(const nanorts_game* game, Shape* out, std::string* why) {
 
 // The first pass's slot window: with more than kSlotWindow slots per player,
 // the first pass stages slots [0, N + kSlotWindow) and the first
-// kSlotWindow of player 1's block only (KGame::shift).  Slots are taken
+// kSlotWindow of player 1's block only (KGame::shift; up to twice as many with
+// one game per wave, see shape_for_first_pass).  Slots are taken
 // lowest-free-first, so a player's units sit at the bottom of its block; a
 // game holding a unit outside the window, or where a spawn could land
 // there, goes to the second pass.  On basesWorkers16x16 (70 slots a player)
@@ -1928,7 +1929,7 @@ NR_DEV void rollout_cycles(const RolloutArgs& args) {
     uint32_t ek0 = (uint32_t)tuni<TW>(e.sc[S_ROOT0]), ek1 = (uint32_t)tuni<TW>(e.sc[S_ROOT1]);
     fold_in(ek0, ek1, (uint32_t)tuni<TW>(e.sc[S_EPISODE]));
     const int32_t steps = args.steps;
-    int32_t general = 0;  // cycles admitted request by request
+    int32_t general = 0;  // cycles of the general admission
     int32_t stop = steps;  // first pass: the first cycle left to the second
     // the output rows of the launch's first cycle and the observation ring,
     // read once into registers instead of from the argument segment every
@@ -2145,10 +2146,10 @@ __global__ __launch_bounds__(256, 4) void k_rollout(RolloutArgs args) { rollout_
 __global__ __launch_bounds__(256, 4) void k_rollout_spanned(RolloutArgs args) { rollout_cycles<false>(args); }
 
 // The first pass: the one-wave path alone, on a smaller LDS block per game.
-// Without the request-by-request admission and completion's member records
-// its code is smaller and keeps fewer scalar registers (90 VGPRs, 60 SGPRs
-// spilled to VGPR lanes against k_rollout's 112 and 117), which makes a
-// cycle about 2.5 % faster at the same 16 games per CU.
+// Without the general admission and completion's member records its code is
+// smaller and keeps fewer registers (102 VGPRs, 96 SGPRs spilled to VGPR lanes
+// against k_rollout's 126 and 136), which made a cycle about 2.5 % faster at the
+// same 16 games per CU.
 __global__ __launch_bounds__(kWave * kLeanMaxGames) void k_rollout_lean(RolloutArgs args) {
     rollout_cycles<true>(args);
 }
@@ -2157,7 +2158,7 @@ __global__ __launch_bounds__(kWave * kLeanMaxGames) void k_rollout_lean(RolloutA
 // runs one game's cycles, so the phases whose work is narrower than a wave
 // (sampling, admission, completion, the slot pass) serve two games per
 // instruction.  A game leaves for the second pass at the first cycle with
-// more than 32 available units or live slots.
+// more than 32 available units or 64 live slots.
 __global__ __launch_bounds__(kWave * kPairMaxWaves, 4) void k_rollout_pair(RolloutArgs args) {
     rollout_cycles<true, 32>(args);
 }
@@ -3736,7 +3737,7 @@ static int env_step(void* stream, const nanorts_game* game, const nanorts_state&
     // second steps what the first left.
     Shape pair;
     std::string why;
-    const ForcedPass forced = forced_first_pass();
+    const ForcedPass forced = taken ? forced_first_pass() : ForcedPass::kNone;
     const bool asked = forced == ForcedPass::kPair;
     bool most = false;
     const bool paired = taken && lanes > 0 && forced != ForcedPass::kLean &&

@@ -614,8 +614,8 @@ class NanoRTS:
     def rollout_first_pass(self) -> str | None:
         """The first pass rollout() runs on this game (with two_pass) where
         the games fill the device: "pair" (two games per wave), "lean" (one
-        game per wave, also for a rollout of few games) or None (one pass on
-        the full block).  The environment variable NANORTS_AMD_FIRST_PASS
+        game per wave, on most boards also for a rollout of few games) or
+        None (one pass on the full block).  The environment variable NANORTS_AMD_FIRST_PASS
         ("lean" or "pair") overrides the library's choice by board."""
         code = self.lib.nanorts_amd_rollout_first_pass(self.dev.ref)
         if code < 0:
@@ -628,7 +628,7 @@ class NanoRTS:
         """Fused rollout: `steps` cycles of masks -> sample -> env.step with the
         state resident in LDS, in place.  Bit-equal to the per-call API.  With
         count_general, out["general_admissions"] int32[L] counts each env's
-        cycles that took the request-at-a-time admission.  With two_pass (the
+        cycles that took the general admission.  With two_pass (the
         default), each launch first runs the games on a smaller LDS block
         and hands the cycles that need the full block to a second pass;
         out["first_pass_cycles"] int32[L] holds the cycles of the last launch

@@ -312,7 +312,7 @@ def _crowded(game, L: int, units0: int = 72, units1: int = 12, seed: int = 5) ->
 
 def test_crowded_rollout_takes_the_general_admission(oracle_threads):
     """With more than 64 available units a cycle's requests do not fit one
-    wave, and the fused rollout admits them request by request.  The
+    wave, and the fused rollout takes the general admission.  The
     rollout's own count shows that path ran in every game, and the result
     matches the oracle."""
     from oracle.oracle import Oracle
