@@ -58,7 +58,8 @@ def crowded_start(game, L, seed=3):
 @pytest.mark.parametrize("name,strategy,partial", [
     ("basesWorkers8x8", "CANCEL_ALTERNATING", False), ("basesWorkers16x16", "CANCEL_ALTERNATING", True),
     ("basesWorkers16x16", "CANCEL_BOTH", False), ("letMeOut", "CANCEL_RANDOM", True),
-    ("basesWorkers24x24A", "CANCEL_RANDOM", True), ("basesWorkers32x32A", "CANCEL_BOTH", True)])
+    ("basesWorkers24x24A", "CANCEL_RANDOM", True), ("basesWorkers32x32A", "CANCEL_BOTH", True),
+    ("GardenOfWar64x64", "CANCEL_RANDOM", True)])
 def test_two_passes_match_oracle(name, strategy, partial, monkeypatch, oracle_threads):
     """Every output and the whole state of each step against the oracle, over
     the horizon (final observations, resets), with an odd number of games."""
